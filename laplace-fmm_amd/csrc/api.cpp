@@ -34,6 +34,16 @@ constexpr int kMixedFirstLevel = 4;
 // direction-split launch over all parents.
 constexpr int64_t kBucketMinParents = 4096;
 
+// FP64 M2L on the vector units: levels of at least this many boxes with on
+// average this many children per parent are packed class-major first.  The
+// pass reads and writes a level's multipoles once (0.2 ms at 262,144 boxes and
+// 13 terms, where it takes the M2L from 20.1 to 17.4 ms); the packed copy
+// holds 8 children per parent, so half-empty levels would write more than
+// they save (1M clustered particles, 13 terms: 10.0 ms with and without at 2
+// to 4 children per parent).
+constexpr int64_t kPackMinBoxes = 4096;
+constexpr int kPackMinFill = 4;
+
 int get_tables(lfmm_ctx* ctx, int N, const DevTables** out)
 {
     auto it = ctx->tables.find(N);
@@ -47,7 +57,17 @@ int get_tables(lfmm_ctx* ctx, int N, const DevTables** out)
     const size_t b_dt = T.dir_theta.size() * 4, b_dtr = T.dir_trans.size() * 4, b_dv = T.dir_vec.size() * 4,
                  b_cd = T.class_dirs.size() * 4, b_k = T.knm.size() * 8;
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t total = al(b_rot) + al(b_eph) + al(b_tr) + al(b_dt) + al(b_dtr) + al(b_dv) + al(b_cd) + al(b_k);
+    M2LSteps MS;
+    pack_m2l_steps(T, MS);
+    M64Pack M;
+    M2lvPack V;
+    if (N <= kM2lvMaxTerms) pack_m2lv(T, V);
+    else pack_m2l64(T, M);
+    const std::vector<double> zero(2 * (size_t)tri(N), 0.0);
+    const size_t b_mr = M.rot.size() * 8, b_mt = M.trans.size() * 8, b_me = M.ephi.size() * 8, b_ms = MS.steps.size() * 4, b_mg = MS.groups.size() * 4,
+                 b_z = zero.size() * 8, b_vr = V.rot.size() * 8, b_vt = V.trans.size() * 8, b_ve = V.ephi.size() * 8;
+    const size_t total = al(b_rot) + al(b_eph) + al(b_tr) + al(b_dt) + al(b_dtr) + al(b_dv) + al(b_cd) + al(b_k) +
+                         al(b_mr) + al(b_mt) + al(b_me) + al(b_ms) + al(b_mg) + al(b_z) + al(b_vr) + al(b_vt) + al(b_ve);
     char* blk = nullptr;
     if (hipMalloc(&blk, total) != hipSuccess) return LFMM_ERR_NOMEM;
     size_t o = 0;
@@ -69,6 +89,16 @@ int get_tables(lfmm_ctx* ctx, int N, const DevTables** out)
     D.rt.dir_vec = (const int*)put(T.dir_vec.data(), b_dv);
     D.rt.class_dirs = (const int*)put(T.class_dirs.data(), b_cd);
     D.knm = (const double*)put(T.knm.data(), b_k);
+    D.m64.rot = (const double2*)put(M.rot.data(), b_mr);
+    D.m64.trans = (const double2*)put(M.trans.data(), b_mt);
+    D.m64.ephi = (const double2*)put(M.ephi.data(), b_me);
+    D.steps.steps = (const int2*)put(MS.steps.data(), b_ms);
+    D.steps.groups = (const int4*)put(MS.groups.data(), b_mg);
+    D.steps.zero = (const double2*)put(zero.data(), b_z);
+    for (int c = 0; c < 8; ++c) D.steps.nsteps[c] = MS.nsteps[c];
+    D.m2lv.rot = (const double*)put(V.rot.data(), b_vr);
+    D.m2lv.trans = (const double*)put(V.trans.data(), b_vt);
+    D.m2lv.ephi = (const double*)put(V.ephi.data(), b_ve);
     if (!copy_ok || hipDeviceSynchronize() != hipSuccess) {
         (void)hipFree(blk);
         return LFMM_ERR_HIP;
@@ -76,6 +106,14 @@ int get_tables(lfmm_ctx* ctx, int N, const DevTables** out)
     auto res = ctx->tables.emplace(N, D);
     *out = &res.first->second;
     return LFMM_OK;
+}
+
+// FP64 M2L (with the L2L) of one level: on the vector units while the step
+// state of 64 targets and two tables fit the LDS, on the matrix cores above.
+static int m2l_fp64_tile(int N) { return N <= kM2lvMaxTerms ? kM2lvTile : m64_tile(N); }
+static hipError_t launch_m2l_fp64(int N, const DevTables& D, const M64Level& A, hipStream_t st)
+{
+    return N <= kM2lvMaxTerms ? launch_m2lv(N, D.steps, D.m2lv, A, st) : launch_m2l64(N, D.steps, D.m64, A, st);
 }
 
 // Split-fp16 dense M2L operators of N terms (m2l_dense.cpp), built once per context.
@@ -649,6 +687,14 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
     // direction parts: levels with fewer workgroups than the chip holds split
     // their 189 directions over more workgroups (deterministic partial sums)
     auto dsplit_for = [](int64_t wgs) { return (int)std::max<int64_t>(1, std::min<int64_t>(32, (1024 + wgs - 1) / wgs)); };
+    double2* vpack = nullptr;  // class-major sources of the FP64 M2L, one buffer for all levels
+    if (far && !per_box && N <= kM2lvMaxTerms) {
+        int64_t big = 0;
+        for (int l = first; l < (mixed ? std::min(mfl, depth) : depth); ++l)
+            if (cnt[l] >= kPackMinBoxes && cnt[l] >= (int64_t)kPackMinFill * cnt[l - 1])
+                big = std::max<int64_t>(big, m2lv_slots(cnt[l - 1]));
+        if (big > 0 && !(vpack = take<double2>(A, 8 * NX * big))) return LFMM_ERR_NOMEM;
+    }
     double2* list_partial = nullptr;  // direction parts of the matrix-core M2L buckets
     int64_t list_partial_elems = 0;
     if (far) {
@@ -666,6 +712,13 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
             L.dst = inner[l];
             L.tiles = (int)((cnt[l - 1] + rtr_tile(N) - 1) / rtr_tile(N));
             const bool bucketed = adaptive && l >= mfl && (per_box || cnt[l - 1] >= kBucketMinParents);
+            // FP64 M2L of a large, mostly full level: sources class-major
+            double2* vpacked = nullptr;
+            if (!(mixed && l >= mfl) && !per_box && N <= kM2lvMaxTerms && cnt[l] >= kPackMinBoxes &&
+                cnt[l] >= (int64_t)kPackMinFill * cnt[l - 1]) {
+                vpacked = vpack;
+                LFMM_HIP(launch_m2lv_pack(L, NX, vpacked, st));
+            }
             if (bucketed) {
                 // the level's sources packed once, at the largest order of its buckets
                 int tpack = 0;
@@ -697,9 +750,10 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                     Lb.dsplit = 1;
                     Lb.csorted = 1;
                     for (int c = 0; c <= 8; ++c) Lb.coff[c] = (int)(O.seg[key + c] - b0);
+                    const int tw = mixed ? rtr_tile(t) : m2l_fp64_tile(t);
                     Lb.ctile[0] = 0;
                     for (int c = 0; c < 8; ++c)
-                        Lb.ctile[c + 1] = Lb.ctile[c] + (Lb.coff[c + 1] - Lb.coff[c] + rtr_tile(t) - 1) / rtr_tile(t);
+                        Lb.ctile[c + 1] = Lb.ctile[c] + (Lb.coff[c + 1] - Lb.coff[c] + tw - 1) / tw;
                     Lb.tiles = Lb.ctile[8];
                     if (mixed) {
                         M2L16Args m{};
@@ -757,7 +811,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                         ++mixed_launches;
                     } else {
                         LFMM_HIP(ev_open());
-                        LFMM_HIP(launch_rtr(t, 1, DB->rt, Lb, st));
+                        LFMM_HIP(launch_m2l_fp64(t, *DB, M64Level{Lb, lut[l - 1], lkeys[l - 1], (int)cnt[l - 1], vpacked, m2lv_slots(cnt[l - 1])}, st));
                         LFMM_HIP(ev_close(EV_M2L64));
                     }
                     ++m2l_launches;
@@ -805,13 +859,14 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                 LFMM_HIP(ev_close(EV_M2L16));
                 ++mixed_launches;
             } else {
+                L.tiles = (int)((cnt[l - 1] + m2l_fp64_tile(N) - 1) / m2l_fp64_tile(N));
                 L.dsplit = dsplit_for((int64_t)L.tiles * 8);
                 if (L.dsplit > 1) {
                     L.partial = take<double2>(A, (int64_t)L.dsplit * cnt[l] * NX);
                     if (!L.partial) return LFMM_ERR_NOMEM;
                 }
                 LFMM_HIP(ev_open());
-                LFMM_HIP(launch_rtr(N, 1, DT->rt, L, st));
+                LFMM_HIP(launch_m2l_fp64(N, *DT, M64Level{L, lut[l - 1], lkeys[l - 1], (int)cnt[l - 1], vpacked, m2lv_slots(cnt[l - 1])}, st));
                 if (L.dsplit > 1) LFMM_HIP(launch_sum_parts(L.partial, L.dsplit, cnt[l] * NX, inner[l], false, st));
                 LFMM_HIP(ev_close(EV_M2L64));
             }

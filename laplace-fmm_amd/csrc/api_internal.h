@@ -4,6 +4,7 @@
 #include "lfmm.h"
 #include "lfmm_internal.h"
 #include "ops3d.h"
+#include "m2lv.h"
 #include "tree.h"
 #include "adaptive.h"
 #include "order.h"
@@ -78,6 +79,9 @@ struct DevTables {
     int N = 0;
     void* block = nullptr;
     RtrTables rt{};
+    M2LStepTables steps{};
+    M64Tables m64{};
+    M2lvTables m2lv{};
     const double* knm = nullptr;
     uint4* m16 = nullptr;      // split-fp16 dense M2L operators (built on first mixed solve)
     const int2* m16_kpre = nullptr;  // their block prefixes (same allocation)

@@ -48,18 +48,18 @@ constexpr int rtr_tile(int N)
 }
 
 struct RtrLevel {
-    int level;                 // M2L: target level; M2M: parent level
-    int num_parents;           // M2L: boxes at level-1; M2M: boxes at level
+    int level;                 // M2L, L2L: target level; M2M: parent level
+    int num_parents;           // M2L, L2L: boxes at level-1; M2M: boxes at level
     const int32_t* child_begin;   // child ranges of those parents
     const uint64_t* child_keys;   // keys of the child level
     const int32_t* lut;        // M2L source lookup at `level` (dense) or null
     const uint64_t* keys;      // keys at `level` (binary search fallback)
     int size;                  // boxes at `level`
     const double2* src;        // M2L: outer[level]; M2M: outer[level+1]
-    const double2* parent_local;  // M2L: inner[level-1] (null: no L2L)
-    double2* dst;              // M2L: inner[level]; M2M: outer[level]
-    // M2L / L2L: target tiles (ceil(num_parents / rtr_tile(N))) and the number
-    // of direction parts; with dsplit > 1 part p writes partial + p*size*NX
+    const double2* parent_local;  // M2L, L2L: inner[level-1] (M2L: null without L2L)
+    double2* dst;              // M2L, L2L: inner[level]; M2M: outer[level]
+    // M2L / L2L: target tiles (ceil(num_parents / targets per workgroup of the
+    // kernel)) and the number of direction parts; with dsplit > 1 part p writes partial + p*size*NX
     // and a reduction forms dst (small levels: more workgroups than tiles).
     int tiles = 0;
     int dsplit = 1;
@@ -72,7 +72,7 @@ struct RtrLevel {
     int stride = 0;
     // class-sorted parent list (M2L / L2L with plist): the parents with a
     // class-c child are plist[coff[c] .. coff[c+1]), and blocks
-    // ctile[c] .. ctile[c+1] serve them (tiles of rtr_tile(N) parents)
+    // ctile[c] .. ctile[c+1] serve them (tiles of the kernel's targets)
     int csorted = 0;
     int coff[9] = {};
     int ctile[9] = {};

@@ -2,7 +2,8 @@
 // Compiled once per expansion size by ops3d_inst.hip (-DLFMM_N=<terms>).
 //
 //   k_p2m   P2M, wave per leaf           (reference Multipole, src/cpu/multipole3d.cpp:20-49)
-//   k_rtr   M2M and M2L(+L2L)            (reference M2M :115-150, M2L :152-190, L2L :192-226)
+//   k_rtr   M2M and L2L                  (reference M2M :115-150, L2L :192-226); the M2L is in
+//           m2lv_kernels.h, m2l64_kernels.h (FP64) and m2l16_kernels.h (split FP16)
 //   k_l2p   L2P, lane per target particle, far field in sorted order
 //           (reference ComputeLeaves<double> :1156-1210); the pair sums and the
 //           scatter to input order are in p2p.hip
@@ -12,8 +13,9 @@
 //
 // k_rtr is the rotate / axial-translate / rotate-back operator.  A workgroup
 // of 4 waves owns 64 target boxes (one per lane, the same lane in every
-// wave) and walks the interaction directions in lock step, so all rotation
-// and translation coefficients of a step are wave-uniform (scalar loads).
+// wave) and walks its directions (M2M: the 8 child classes; L2L: one) in lock
+// step, so all rotation and translation coefficients of a step are
+// wave-uniform (scalar loads).
 // Per direction the op state (one expansion per lane) lives in LDS as
 // [coefficient][lane] and is produced / consumed in three phases that are
 // partitioned over the 4 waves in three different ways:
@@ -279,10 +281,10 @@ __global__ void __launch_bounds__(256) k_p2m(P2MArgs a, const double* __restrict
 }
 
 // ===================================================================== rotate-translate-rotate
-enum { KIND_M2M = 0, KIND_M2L = 1, KIND_L2L = 2 };  // KIND_L2L: the L2L step of KIND_M2L alone
+enum { KIND_M2M = 0, KIND_L2L = 2 };
 
 // rtr_tile(N) (targets per workgroup) is declared in ops3d.h.
-enum { TR_M2L = 0, TR_M2M = 1, TR_L2L = 2 };
+enum { TR_M2M = 1, TR_L2L = 2 };
 
 template <int N, int W, int TK>
 __device__ __forceinline__ void rtr_phase_b(const double* __restrict__ tt, double2* lds, int lane)
@@ -305,7 +307,7 @@ __device__ __forceinline__ void rtr_phase_b(const double* __restrict__ tt, doubl
                 double yr = 0.0, yi = 0.0;
                 sfor<0, L>([&](auto I) {
                     constexpr int i = decltype(I)::value;
-                    constexpr bool nz = (TK == TR_M2L) || (TK == TR_M2M && i <= j) || (TK == TR_L2L && i >= j);
+                    constexpr bool nz = TK == TR_M2M ? i <= j : i >= j;
                     if constexpr (nz) {
                         const double c = t[j * L + i];
                         yr = fma(c, x[i].x, yr);
@@ -323,9 +325,8 @@ __device__ __forceinline__ void rtr_phase_b(const double* __restrict__ tt, doubl
 // with scalar loads.
 #define RTR_TABLE_PARAMS                                                                             \
     const double2* __restrict__ Trot, const double2* __restrict__ Tephi, const double* __restrict__ Ttrans, \
-        const int* __restrict__ Tdir_theta, const int* __restrict__ Tdir_trans, const int* __restrict__ Tdir_vec, \
-        const int* __restrict__ Tclass_dirs
-#define RTR_TABLE_ARGS Trot, Tephi, Ttrans, Tdir_theta, Tdir_trans, Tdir_vec, Tclass_dirs
+        const int* __restrict__ Tdir_theta
+#define RTR_TABLE_ARGS Trot, Tephi, Ttrans, Tdir_theta
 
 // Barrier for LDS hand-over between the phases: waits for this wave's LDS
 // traffic only, so global prefetch loads stay in flight across it.
@@ -349,7 +350,6 @@ struct PrefetchLayout {
 struct RtrStep {
     int sidx;                 // source box for this lane (-1: none)
     int dir;                  // direction table index
-    int tk;                   // translation kind
     const double2* src;       // source expansion array
 };
 
@@ -406,28 +406,19 @@ __device__ __forceinline__ void rtr_wave(RTR_TABLE_PARAMS, const RtrLevel& L, do
         ce = L.child_begin[P + 1];
     }
     int tgt = -1;
-    uint32_t tx = 0, ty = 0, tz = 0;
     if constexpr (KIND != KIND_M2M) {
         for (int i = cb; i < ce; ++i)
             if ((int)(L.child_keys[i] & 7u) == c) tgt = i;
-        if (tgt >= 0) {
-            const uint64_t k = L.child_keys[tgt];
-            tx = compact3(k >> 2);
-            ty = compact3(k >> 1);
-            tz = compact3(k);
-        }
     } else {
         // a parent without children (a leaf of the adaptive tree) keeps its P2M
         tgt = (pvalid && ce > cb) ? P : -1;
     }
-    const int side = 1 << L.level;
     double2 acc[NX];
 #pragma unroll
     for (int i = 0; i < NX; ++i) acc[i] = make_double2(0.0, 0.0);
 
-    const int has_l2l = (KIND == KIND_L2L || (KIND == KIND_M2L && L.parent_local)) ? 1 : 0;
-    const int ndir = (KIND == KIND_M2M) ? 8 : (KIND == KIND_L2L ? 1 : kDirsPerClass + has_l2l);
-    // directions [d_beg, d_end) of this part (L.dsplit parts; the L2L step is in part 0)
+    const int ndir = KIND == KIND_M2M ? 8 : 1;
+    // directions [d_beg, d_end) of this part (L.dsplit parts)
     const int d_beg = (int)((int64_t)part * ndir / L.dsplit), d_end = (int)((int64_t)(part + 1) * ndir / L.dsplit);
 
     auto step_of = [&](int d) {
@@ -435,27 +426,13 @@ __device__ __forceinline__ void rtr_wave(RTR_TABLE_PARAMS, const RtrLevel& L, do
         s.sidx = -1;
         if constexpr (KIND == KIND_M2M) {
             s.dir = kDiagBase + d;
-            s.tk = TR_M2M;
             s.src = L.src;
             for (int i = cb; i < ce; ++i)
                 if ((int)(L.child_keys[i] & 7u) == d) s.sidx = i;
         } else {
-            if (has_l2l && d == 0) {
-                s.dir = kDiagBase + (7 - c);
-                s.tk = TR_L2L;
-                s.src = L.parent_local;
-                s.sidx = tgt >= 0 ? P : -1;
-            } else {
-                s.dir = Tclass_dirs[c * kDirsPerClass + (d - has_l2l)];
-                s.tk = TR_M2L;
-                s.src = L.src;
-                if (tgt >= 0) {
-                    const int sx = (int)tx + Tdir_vec[4 * s.dir], sy = (int)ty + Tdir_vec[4 * s.dir + 1],
-                              sz = (int)tz + Tdir_vec[4 * s.dir + 2];
-                    if (sx >= 0 && sy >= 0 && sz >= 0 && sx < side && sy < side && sz < side)
-                        s.sidx = find_box(morton3(sx, sy, sz), L.lut, L.keys, L.size);
-                }
-            }
+            s.dir = kDiagBase + (7 - c);
+            s.src = L.parent_local;
+            s.sidx = tgt >= 0 ? P : -1;
         }
         return s;
     };
@@ -509,16 +486,8 @@ __device__ __forceinline__ void rtr_wave(RTR_TABLE_PARAMS, const RtrLevel& L, do
             });
             lds_barrier();
             // ---- phase B: axial translation, by order
-            const int tsel = (cur.tk == TR_M2L) ? Tdir_trans[cur.dir] : (cur.tk == TR_M2M ? kTransM2M : kTransL2L);
-            const double* __restrict__ tt = Ttrans + (int64_t)tsel * TS;
-            if constexpr (KIND == KIND_M2M) {
-                rtr_phase_b<N, W, TR_M2M>(tt, lds, lane);
-            } else if constexpr (KIND == KIND_L2L) {
-                rtr_phase_b<N, W, TR_L2L>(tt, lds, lane);
-            } else {
-                if (cur.tk == TR_L2L) rtr_phase_b<N, W, TR_L2L>(tt, lds, lane);
-                else rtr_phase_b<N, W, TR_M2L>(tt, lds, lane);
-            }
+            const double* __restrict__ tt = Ttrans + (int64_t)(KIND == KIND_M2M ? kTransM2M : kTransL2L) * TS;
+            rtr_phase_b<N, W, KIND == KIND_M2M ? TR_M2M : TR_L2L>(tt, lds, lane);
             lds_barrier();
         }
         // issue the next step's source loads; they complete under phase C
@@ -784,6 +753,7 @@ template <int N>
 hipError_t do_rtr(int kind, const RtrTables& T, const RtrLevel& L, hipStream_t st)
 {
     const int tiles = (L.num_parents + rtr_tile(N) - 1) / rtr_tile(N);
+    if (kind != KIND_M2M && kind != KIND_L2L) return hipErrorInvalidValue;
     if (tiles == 0) return hipSuccess;
     if (L.tiles != tiles && kind != KIND_M2M && !L.csorted) return hipErrorInvalidValue;
     if (L.csorted && kind != KIND_M2M) {
@@ -794,23 +764,15 @@ hipError_t do_rtr(int kind, const RtrTables& T, const RtrLevel& L, hipStream_t s
         int mt = 0;
         for (int c = 0; c < 8; ++c) mt = std::max(mt, L.ctile[c + 1] - L.ctile[c]);
         if (mt == 0) return hipSuccess;
-        if (kind == KIND_L2L)
-            hipLaunchKernelGGL((k_rtr<N, KIND_L2L>), dim3(8 * mt), dim3(256), 0, st, T.rot, T.ephi, T.trans,
-                               T.dir_theta, T.dir_trans, T.dir_vec, T.class_dirs, L);
-        else
-            hipLaunchKernelGGL((k_rtr<N, KIND_M2L>), dim3(8 * mt), dim3(256), 0, st, T.rot, T.ephi, T.trans,
-                               T.dir_theta, T.dir_trans, T.dir_vec, T.class_dirs, L);
+        hipLaunchKernelGGL((k_rtr<N, KIND_L2L>), dim3(8 * mt), dim3(256), 0, st, T.rot, T.ephi, T.trans, T.dir_theta, L);
         return hipGetLastError();
     }
     if (kind == KIND_M2M)
         hipLaunchKernelGGL((k_rtr<N, KIND_M2M>), dim3(tiles * L.dsplit), dim3(256), 0, st, T.rot, T.ephi, T.trans,
-                           T.dir_theta, T.dir_trans, T.dir_vec, T.class_dirs, L);
-    else if (kind == KIND_L2L)
-        hipLaunchKernelGGL((k_rtr<N, KIND_L2L>), dim3(tiles * 8 * L.dsplit), dim3(256), 0, st, T.rot, T.ephi, T.trans,
-                           T.dir_theta, T.dir_trans, T.dir_vec, T.class_dirs, L);
+                           T.dir_theta, L);
     else
-        hipLaunchKernelGGL((k_rtr<N, KIND_M2L>), dim3(tiles * 8 * L.dsplit), dim3(256), 0, st, T.rot, T.ephi, T.trans,
-                           T.dir_theta, T.dir_trans, T.dir_vec, T.class_dirs, L);
+        hipLaunchKernelGGL((k_rtr<N, KIND_L2L>), dim3(tiles * 8 * L.dsplit), dim3(256), 0, st, T.rot, T.ephi, T.trans,
+                           T.dir_theta, L);
     return hipGetLastError();
 }
 
