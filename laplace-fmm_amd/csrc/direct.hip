@@ -3,8 +3,7 @@
 // pair terms of src/common/simple_math.h:120-151 and their device forms
 // :197-208).
 //
-// One thread per target; sources stream through LDS in tiles of 256 packed
-// (x, y, z, q) records, each added in input order.  3D pair:
+// 3D pair:
 //   q / max(|r|, 1e-4)  and  q r / max(|r|, 1e-4)^3   (r = x_i - x_j)
 // evaluated as q * rsqrt(max(|r|^2, 1e-8)), the reference's device form.
 // 2D pair: q * 0.5 log max(|dz|^2, 1e-8) and q conj(dz) / max(|dz|^2, 1e-8).
@@ -21,85 +20,134 @@ namespace {
 
 constexpr int kTile = 256;
 
-// 1 / sqrt(r2): v_rsq_f64 refined by two Newton steps (full FP64 accuracy)
+// 1 / sqrt(r2): v_rsq_f64 (relative error 5e-8) refined by one third-order
+// step: with e = 1 - r2 y^2, y (1 + e / 2 + 3 e^2 / 8) leaves 5/16 e^3, far
+// below the rounding of the last operation
 __device__ __forceinline__ double rsqrt_full(double r2)
 {
-    double y = __builtin_amdgcn_rsq(r2);
-    const double hr = 0.5 * r2;
-    y = y * fma(-hr * y, y, 1.5);
-    y = y * fma(-hr * y, y, 1.5);
-    return y;
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double e = fma(-(r2 * y), y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-__global__ void __launch_bounds__(kTile) k_direct3d(const double4* __restrict__ tgt, int64_t nt,
-                                                   const double4* __restrict__ src, int64_t ns, int exclude,
-                                                   double* __restrict__ pot, double* __restrict__ field)
-{
-    __shared__ double4 tile[kTile];
-    const int64_t i = (int64_t)blockIdx.x * kTile + threadIdx.x;
-    const double4 t = i < nt ? tgt[i] : make_double4(0.0, 0.0, 0.0, 0.0);
+// All pairs.  A workgroup of 1024 threads owns 2 LT targets, two per lane
+// (LT lanes), and cuts the sources into 1024 / LT interleaved slices, one per
+// group of LT lanes; the slices' sums are added in a fixed order at the end
+// (shuffles within a wave, then LDS over the waves).  So few targets still
+// fill the chip without a buffer for partial sums: one thread per target ran
+// 4,096 targets on 16 of 256 CUs (123 ms against 1,048,576 sources).
+// Bound by FP64 vector issue: 23 operations and v_rsq_f64 per 3D pair.  With
+// LT >= 64 a wave's source is uniform and arrives by scalar loads; below, two
+// targets per lane halve the L1 reads per pair, which one target per lane
+// would be bound by (64 lanes x 32 bytes at 64 bytes per cycle).
+template <int DIM>
+struct DirectSum;
+template <>
+struct DirectSum<3> {
     double p = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
-    for (int64_t base = 0; base < ns; base += kTile) {
-        __syncthreads();
-        const int64_t j0 = base + threadIdx.x;
-        tile[threadIdx.x] = j0 < ns ? src[j0] : make_double4(0.0, 0.0, 0.0, 0.0);
-        __syncthreads();
-        const int cnt = (int)min<int64_t>(kTile, ns - base);
-        for (int j = 0; j < cnt; ++j) {
-            if (exclude && base + j == i) continue;
-            const double4 s = tile[j];
-            const double dx = t.x - s.x, dy = t.y - s.y, dz = t.z - s.z;
-            const double r2 = fmax(fma(dx, dx, fma(dy, dy, dz * dz)), 1.e-8);
-            const double ir = rsqrt_full(r2);
-            const double qi = s.w * ir;
-            p += qi;
-            const double q3 = qi * ir * ir;
-            fx = fma(q3, dx, fx);
-            fy = fma(q3, dy, fy);
-            fz = fma(q3, dz, fz);
-        }
+    __device__ __forceinline__ void add(const double4& t, double sx, double sy, double sz, double q)
+    {
+        const double dx = t.x - sx, dy = t.y - sy, dz = t.z - sz;
+        const double r2 = fmax(fma(dx, dx, fma(dy, dy, dz * dz)), 1.e-8);
+        const double ir = rsqrt_full(r2);
+        const double qi = q * ir;
+        p += qi;
+        const double q3 = qi * (ir * ir);
+        fx = fma(q3, dx, fx);
+        fy = fma(q3, dy, fy);
+        fz = fma(q3, dz, fz);
     }
-    if (i < nt) {
-        if (pot) pot[i] = p;
-        if (field) {
-            field[3 * i] = fx;
-            field[3 * i + 1] = fy;
-            field[3 * i + 2] = fz;
-        }
+};
+template <>
+struct DirectSum<2> {
+    double p = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;  // fz unused
+    __device__ __forceinline__ void add(const double4& t, double sx, double sy, double, double q)
+    {
+        // packed 2D records are (x, y, 0, q)
+        const double dx = t.x - sx, dy = t.y - sy;
+        const double r2 = fmax(fma(dx, dx, dy * dy), 1.e-8);
+        p = fma(q * 0.5, log(r2), p);
+        const double qr = q / r2;
+        fx = fma(qr, dx, fx);
+        fy = fma(-qr, dy, fy);
     }
-}
+};
 
-__global__ void __launch_bounds__(kTile) k_direct2d(const double4* __restrict__ tgt, int64_t nt,
-                                                   const double4* __restrict__ src, int64_t ns, int exclude,
-                                                   double* __restrict__ pot, double* __restrict__ field)
+constexpr int kDirectThreads = 1024;
+
+template <int DIM, int LT, bool EXCLUDE>
+__global__ void __launch_bounds__(kDirectThreads) k_direct(const double4* __restrict__ tgt, int64_t nt,
+                                                          const double4* __restrict__ src, int64_t ns,
+                                                          double* __restrict__ pot, double* __restrict__ field)
 {
-    __shared__ double4 tile[kTile];
-    const int64_t i = (int64_t)blockIdx.x * kTile + threadIdx.x;
-    const double4 t = i < nt ? tgt[i] : make_double4(0.0, 0.0, 0.0, 0.0);
-    double p = 0.0, fx = 0.0, fy = 0.0;
-    for (int64_t base = 0; base < ns; base += kTile) {
-        __syncthreads();
-        const int64_t j0 = base + threadIdx.x;
-        tile[threadIdx.x] = j0 < ns ? src[j0] : make_double4(0.0, 0.0, 0.0, 0.0);
-        __syncthreads();
-        const int cnt = (int)min<int64_t>(kTile, ns - base);
-        for (int j = 0; j < cnt; ++j) {
-            if (exclude && base + j == i) continue;
-            const double4 s = tile[j];
-            // packed 2D records are (x, y, 0, q)
-            const double dx = t.x - s.x, dy = t.y - s.y;
-            const double r2 = fmax(fma(dx, dx, dy * dy), 1.e-8);
-            p = fma(s.w * 0.5, log(r2), p);
-            const double qr = s.w / r2;
-            fx = fma(qr, dx, fx);
-            fy = fma(-qr, dy, fy);
+    constexpr int S = kDirectThreads / LT, NW = kDirectThreads / 64;
+    // per wave the sums of its targets (LT <= 64: 2 LT; above: 2 per lane)
+    constexpr int WT = LT < 64 ? LT : 64;
+    __shared__ double4 part[S > 1 ? 2 * NW * WT : 1];
+    const int lt = threadIdx.x & (LT - 1), lane = threadIdx.x & 63;
+    int64_t i[2];
+    double4 t[2];
+    DirectSum<DIM> a[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        i[u] = (int64_t)blockIdx.x * (2 * LT) + u * LT + lt;
+        t[u] = i[u] < nt ? tgt[i[u]] : make_double4(0.0, 0.0, 0.0, 0.0);
+    }
+    auto pair = [&](int64_t j, double sx, double sy, double sz, double q) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) a[u].add(t[u], sx, sy, sz, EXCLUDE && j == i[u] ? 0.0 : q);
+    };
+    if constexpr (LT >= 64) {
+        typedef const double __attribute__((address_space(4))) scalar;
+        scalar* p = (scalar*)(uintptr_t)src;
+        const int s = __builtin_amdgcn_readfirstlane((int)threadIdx.x / LT);
+#pragma unroll 4
+        for (int64_t j = s; j < ns; j += S) pair(j, p[4 * j], p[4 * j + 1], p[4 * j + 2], p[4 * j + 3]);
+    } else {
+#pragma unroll 4
+        for (int64_t j = threadIdx.x / LT; j < ns; j += S) {
+            const double4 r = src[j];
+            pair(j, r.x, r.y, r.z, r.w);
         }
     }
-    if (i < nt) {
-        if (pot) pot[i] = p;
+    if constexpr (S > 1) {
+        // slices of one wave, then the waves in order
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            for (int off = 32; off >= WT; off >>= 1) {
+                a[u].p += __shfl_xor(a[u].p, off);
+                a[u].fx += __shfl_xor(a[u].fx, off);
+                a[u].fy += __shfl_xor(a[u].fy, off);
+                if constexpr (DIM == 3) a[u].fz += __shfl_xor(a[u].fz, off);
+            }
+            if (lane < WT)
+                part[((threadIdx.x >> 6) * 2 + u) * WT + lane] = make_double4(a[u].p, a[u].fx, a[u].fy, a[u].fz);
+        }
+        __syncthreads();
+        if (threadIdx.x >= LT) return;
+        // wave w holds target lanes (w WT) mod LT ..
+        constexpr int STEP = LT <= 64 ? 1 : LT / 64;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            a[u] = DirectSum<DIM>();
+#pragma unroll 1
+            for (int w = LT <= 64 ? 0 : (int)(threadIdx.x >> 6); w < NW; w += STEP) {
+                const double4 v = part[(w * 2 + u) * WT + (lt & (WT - 1))];
+                a[u].p += v.x;
+                a[u].fx += v.y;
+                a[u].fy += v.z;
+                a[u].fz += v.w;
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        if (i[u] >= nt) continue;
+        if (pot) pot[i[u]] = a[u].p;
         if (field) {
-            field[2 * i] = fx;
-            field[2 * i + 1] = fy;
+            field[DIM * i[u]] = a[u].fx;
+            field[DIM * i[u] + 1] = a[u].fy;
+            if constexpr (DIM == 3) field[DIM * i[u] + 2] = a[u].fz;
         }
     }
 }
@@ -189,16 +237,39 @@ hipError_t launch_cross_fields(const double* e1, const double* e2, double* e3, i
     return hipGetLastError();
 }
 
+template <int DIM, int LT>
+static hipError_t direct_lt(const double4* tgt, int64_t nt, const double4* src, int64_t ns, bool exclude, double* pot,
+                            double* field, hipStream_t st)
+{
+    const dim3 grid((unsigned)((nt + 2 * LT - 1) / (2 * LT)));
+    if (exclude)
+        hipLaunchKernelGGL((k_direct<DIM, LT, true>), grid, dim3(kDirectThreads), 0, st, tgt, nt, src, ns, pot, field);
+    else
+        hipLaunchKernelGGL((k_direct<DIM, LT, false>), grid, dim3(kDirectThreads), 0, st, tgt, nt, src, ns, pot, field);
+    return hipGetLastError();
+}
+
+template <int DIM>
+static hipError_t direct_dim(const double4* tgt, int64_t nt, const double4* src, int64_t ns, bool exclude, double* pot,
+                             double* field, hipStream_t st)
+{
+    // the most targets per workgroup that still give every CU one workgroup
+    int lt = 1;
+    while (lt < kDirectThreads && nt >= (int64_t)256 * 2 * (2 * lt)) lt *= 2;
+    switch (lt) {
+#define X(n) case n: return direct_lt<DIM, n>(tgt, nt, src, ns, exclude, pot, field, st);
+        X(1) X(2) X(4) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
+#undef X
+    default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t launch_direct(int dim, const double4* tgt, int64_t nt, const double4* src, int64_t ns, bool exclude_self,
                          double* pot, double* field, hipStream_t st)
 {
     if (nt <= 0) return hipSuccess;
-    const dim3 grid((unsigned)((nt + kTile - 1) / kTile));
-    if (dim == 3)
-        hipLaunchKernelGGL(k_direct3d, grid, dim3(kTile), 0, st, tgt, nt, src, ns, exclude_self ? 1 : 0, pot, field);
-    else
-        hipLaunchKernelGGL(k_direct2d, grid, dim3(kTile), 0, st, tgt, nt, src, ns, exclude_self ? 1 : 0, pot, field);
-    return hipGetLastError();
+    return dim == 3 ? direct_dim<3>(tgt, nt, src, ns, exclude_self, pot, field, st)
+                    : direct_dim<2>(tgt, nt, src, ns, exclude_self, pot, field, st);
 }
 
 int direct3d_split_count(int64_t nt, int64_t ns)
