@@ -545,23 +545,54 @@ __global__ void __launch_bounds__(256) k_count_p2p(const uint64_t* __restrict__ 
 }
 
 // ------------------------------------------------------------------ near-field ranges
+// Half a wave per leaf: lane o < 27 finds the particle range of neighbour o;
+// the ranges are then put in particle order and runs that touch are joined
+// (Morton order: 27 neighbours make 9 to 10 runs on a full tree), so the pair
+// loop changes ranges a third as often and never meets an empty one.  Unused
+// entries of the leaf's 27 are (0, 0).
 __global__ void __launch_bounds__(256) k_leaf_ranges(const uint64_t* __restrict__ leaf_key,
                                                      const int32_t* __restrict__ leaf_begin, int nleaf, int level,
                                                      const int32_t* __restrict__ lut, int2* __restrict__ nbr)
 {
-    const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (g >= (int64_t)nleaf * 27) return;
-    const int leaf = (int)(g / 27), o = (int)(g % 27);
-    const uint64_t k = leaf_key[leaf];
-    const int x = (int)compact3(k >> 2) + o / 9 - 1, y = (int)compact3(k >> 1) + (o / 3) % 3 - 1,
-              z = (int)compact3(k) + o % 3 - 1;
-    const int side = 1 << level;
-    int2 r = make_int2(0, 0);
-    if (x >= 0 && y >= 0 && z >= 0 && x < side && y < side && z < side) {
-        const int j = (o == 13) ? leaf : lookup(morton3(x, y, z), lut, leaf_key, nleaf);
-        if (j >= 0) r = make_int2(leaf_begin[j], leaf_begin[j + 1]);
+    __shared__ int2 sorted[8][32];
+    const int half = threadIdx.x >> 5, o = threadIdx.x & 31;
+    const int leaf = blockIdx.x * 8 + half;
+    constexpr int kNone = 0x7fffffff;
+    int2 r = make_int2(kNone, kNone);
+    if (leaf < nleaf && o < 27) {
+        const uint64_t k = leaf_key[leaf];
+        const int x = (int)compact3(k >> 2) + o / 9 - 1, y = (int)compact3(k >> 1) + (o / 3) % 3 - 1,
+                  z = (int)compact3(k) + o % 3 - 1;
+        const int side = 1 << level;
+        if (x >= 0 && y >= 0 && z >= 0 && x < side && y < side && z < side) {
+            const int j = (o == 13) ? leaf : lookup(morton3(x, y, z), lut, leaf_key, nleaf);
+            if (j >= 0) r = make_int2(leaf_begin[j], leaf_begin[j + 1]);
+        }
     }
-    nbr[g] = r;
+    // rank among the leaf's ranges (begins are distinct, absent ones last)
+    int rank = 0;
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+        const int bj = __shfl(r.x, j, 32);
+        rank += (bj < r.x || (bj == r.x && j < o)) ? 1 : 0;
+    }
+    sorted[half][rank] = r;
+    __syncthreads();
+    r = sorted[half][o];
+    const bool ok = r.x != kNone;
+    const bool head = ok && (o == 0 || sorted[half][o - 1].y != r.x);
+    const bool tail = ok && (o == 31 || sorted[half][o + 1].x != r.y);
+    const uint32_t heads = (uint32_t)(__ballot(head) >> (threadIdx.x & 32));
+    if (leaf >= nleaf || o >= 27) return;
+    int* out = (int*)(nbr + (int64_t)leaf * 27);
+    const int runs = __popc(heads);
+    const int run = __popc(heads & ((2u << o) - 1u)) - 1;
+    if (head) out[2 * run] = r.x;
+    if (tail) out[2 * run + 1] = r.y;
+    if (o >= runs) {
+        out[2 * o] = 0;
+        out[2 * o + 1] = 0;
+    }
 }
 
 // ================================================================== host side
@@ -771,8 +802,8 @@ hipError_t count_ops(int dim, const std::vector<uint64_t*>& keys, const std::vec
 hipError_t launch_leaf_ranges(const uint64_t* leaf_key, const int32_t* leaf_begin, int nleaf, int level,
                               const int32_t* lut, int2* nbr, hipStream_t st)
 {
-    const int64_t n = (int64_t)nleaf * 27;
-    if (n > 0) hipLaunchKernelGGL(k_leaf_ranges, dim3(nblk(n, 256)), dim3(256), 0, st, leaf_key, leaf_begin, nleaf, level, lut, nbr);
+    if (nleaf > 0)
+        hipLaunchKernelGGL(k_leaf_ranges, dim3(nblk(nleaf, 8)), dim3(256), 0, st, leaf_key, leaf_begin, nleaf, level, lut, nbr);
     return hipGetLastError();
 }
 
