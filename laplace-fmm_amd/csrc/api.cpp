@@ -264,152 +264,137 @@ int build_tree(lfmm_ctx* ctx, const DevPoints& DP, int depth_in, int leaf_max, b
     T.ps = ps;
     T.qs = qs;
 
-    double* geom = take<double>(A, 4);
-    double* part = take<double>(A, 6 * 1024);
-    int* nonfinite = take<int>(A, 1);
-    uint32_t* umax = take<uint32_t>(A, 64);
-    if (!geom || !part || !nonfinite || !umax) return LFMM_ERR_NOMEM;
+    double* geom = take<double>(A, 5);
+    double* part = take<double>(A, 7 * 1024);
+    uint32_t* umax = take<uint32_t>(A, 3);
+    if (!geom || !part || !umax) return LFMM_ERR_NOMEM;
     T.geom = geom;
     T.umax = umax;
     if (fixed_geom) {
         LFMM_HIP(hipMemcpyAsync(geom, fixed_geom, 4 * sizeof(double), hipMemcpyDeviceToDevice, st));
+        LFMM_HIP(hipMemsetAsync(geom + 4, 0, sizeof(double), st));
     } else {
-        LFMM_HIP(hipMemsetAsync(nonfinite, 0, sizeof(int), st));
-        LFMM_HIP(extent(dim, dpos, ps, n, part, nonfinite, geom, st));
-        int bad = 0;
-        LFMM_HIP(hipMemcpyAsync(&bad, nonfinite, sizeof(int), hipMemcpyDeviceToHost, st));
-        LFMM_HIP(hipStreamSynchronize(st));
-        if (bad) return LFMM_ERR_NONFINITE;
+        LFMM_HIP(extent(dim, dpos, ps, n, part, geom, st));
     }
 
     // ---- tree depth (reference rule :1334-1337, or the leaf-size bound)
-    int depth = depth_in;
-    if (depth_in == LFMM_AUTO) {
-        if (leaf_max > 0) {
-            int maxl = 1;
-            while (maxl < lut_max_level(dim) && ((int64_t)1 << (dim * maxl)) < n) ++maxl;
-            int64_t cnt = 0;
-            for (int l = 0; l <= maxl; ++l) cnt += (int64_t)1 << (dim * l);
-            uint32_t* cws = take<uint32_t>(A, cnt);
-            if (!cws) return LFMM_ERR_NOMEM;
-            int lvl = 0;
-            LFMM_HIP(occupancy_depth(dim, dpos, ps, n, geom, leaf_max, maxl, cws, umax, &lvl, st));
-            if (lvl > maxl) {
-                // clustered input: beyond the dense histograms, sort the keys
-                // of the deepest level once and take the largest run of each
-                // coarser key prefix
-                const int deep = dim == 3 ? kMaxDepth - 1 : 2 * kMaxDepth - 2;
-                uint64_t* dk = take<uint64_t>(A, n);
-                uint32_t* dv = take<uint32_t>(A, n);
-                void* dws = A.alloc((size_t)sort_ws_bytes(n));
-                uint32_t* fl = take<uint32_t>(A, n);
-                uint32_t* ex = take<uint32_t>(A, n);
-                uint32_t* sw = take<uint32_t>(A, scan_ws_elems(n));
-                uint64_t* uk = take<uint64_t>(A, n);
-                int32_t* ub = take<int32_t>(A, n + 1);
-                if (!dk || !dv || !dws || !fl || !ex || !sw || !uk || !ub) return LFMM_ERR_NOMEM;
-                LFMM_HIP(keys(dim, dpos, ps, n, deep, geom, dk, dv, st));
-                uint64_t* sk = dk;
-                uint32_t* so = dv;
-                LFMM_HIP(radix_sort(dk, dv, n, dim * deep, dws, st, &sk, &so));
-                lvl = deep;
-                for (int l = maxl + 1; l <= deep; ++l) {
-                    int64_t cnt = 0;
-                    LFMM_HIP(run_compact(sk, n, dim * (deep - l), fl, ex, sw, uk, ub, nullptr, &cnt, st));
-                    uint32_t mx = 0;
-                    LFMM_HIP(max_run(ub, cnt, umax, &mx, st));
-                    if ((int64_t)mx <= leaf_max) {
-                        lvl = l;
-                        break;
-                    }
-                }
-            }
-            depth = lvl + 1;
-        } else if (dim == 3) {  // src/cpu/multipole3d.cpp:1334-1337
-            depth = (int)std::max(2.0, 1 + std::log((double)n / 100.0) / std::log(8.0));
-        } else {                // src/cpu/multipole.cpp:483-487
-            depth = (int)std::max(3.0, 2 + std::log((double)n / 100.0) / std::log(4.0));
-        }
+    const int deepest = dim == 3 ? kMaxDepth - 1 : 2 * kMaxDepth - 2;
+    const bool search = depth_in == LFMM_AUTO && leaf_max > 0;
+    int leaf_level = depth_in - 1;
+    if (search) {
+        // The level is known once keys are in order (keys leaf_max places
+        // apart share a box above it), so the search is a guess to sort by: the
+        // level at which evenly spread particles are sure to fit (five
+        // standard deviations of a box's count), or, for an adaptive tree,
+        // whose input is clustered, the deepest.  A guess one level too fine
+        // (any, for an adaptive tree) keeps its order of the leaves; other
+        // misses sort again.  A histogram of the boxes took 0.17 ms for 4M
+        // particles (one atomic each) and a wait of its own.
+        leaf_level = 0;
+        auto fits = [&](int l) {
+            const double m = (double)n / (double)((int64_t)1 << (dim * l));
+            return m + 5.0 * std::sqrt(m) + 3.0 <= (double)leaf_max;
+        };
+        while (leaf_level < std::min(deepest, lut_max_level(dim)) && !fits(leaf_level)) ++leaf_level;
+        if (keep_parents) leaf_level = deepest;
+    } else if (depth_in == LFMM_AUTO) {
+        if (dim == 3)  // src/cpu/multipole3d.cpp:1334-1337
+            leaf_level = (int)std::max(2.0, 1 + std::log((double)n / 100.0) / std::log(8.0)) - 1;
+        else           // src/cpu/multipole.cpp:483-487
+            leaf_level = (int)std::max(3.0, 2 + std::log((double)n / 100.0) / std::log(4.0)) - 1;
     }
-    depth = std::max(depth, min_depth);
-    if (depth < 1 || depth > (dim == 3 ? kMaxDepth : 2 * kMaxDepth - 1)) return LFMM_ERR_DEPTH;
-    T.depth = depth;
-    const int leaf_level = depth - 1;
+    const int least = min_depth - 1;
+    leaf_level = std::max(leaf_level, least);
+    if (leaf_level < 0 || leaf_level > deepest) return LFMM_ERR_DEPTH;
 
-    // ---- keys and stable sort
+    // ---- keys and stable sort; sizes of the levels, one read
     uint64_t* k0 = take<uint64_t>(A, n);
     uint32_t* v0 = take<uint32_t>(A, n);
     void* sws = A.alloc((size_t)sort_ws_bytes(n));
-    if (!k0 || !v0 || !sws) return LFMM_ERR_NOMEM;
-    LFMM_HIP(keys(dim, dpos, ps, n, leaf_level, geom, k0, v0, st));
+    uint32_t* sums = take<uint32_t>(A, level_tiles(n) * (deepest + 1));
+    T.leaf_of = take<int32_t>(A, n);
+    if (!k0 || !v0 || !sws || !sums || !T.leaf_of) return LFMM_ERR_NOMEM;
     uint64_t* skeys = k0;
     uint32_t* order = v0;
-    if (leaf_level > 0) LFMM_HIP(radix_sort(k0, v0, n, dim * leaf_level, sws, st, &skeys, &order));
-    T.order = order;
-
-    // ---- levels
+    LevelInfo* info = (LevelInfo*)ctx->host_info;
+    int key_level = leaf_level;
+    for (;;) {
+        LFMM_HIP(keys(dim, dpos, ps, n, key_level, geom, k0, v0, umax, st));
+        skeys = k0;
+        order = v0;
+        if (key_level > 0) LFMM_HIP(radix_sort(k0, v0, n, dim * key_level, sws, st, &skeys, &order));
+        LFMM_HIP(count_levels(dim, skeys, n, key_level, search ? leaf_max : 0, sums, geom, umax, info, st));
+        LFMM_HIP(hipStreamSynchronize(st));
+        if (info->geom[4] != 0.0) return LFMM_ERR_NONFINITE;
+        T.max_leaf = info->most[0];
+        if (!search) break;
+        leaf_level = std::max(least, std::min(deepest, (int)info->most[2]));
+        if (leaf_level == key_level) break;
+        if (leaf_level < key_level && leaf_max <= 1024 && (keep_parents || leaf_level == key_level - 1)) {
+            T.max_leaf = info->most[1];  // of an adaptive tree: set with its leaves
+            break;
+        }
+        // too coarse: only the deepest keys tell; too fine: the level is known
+        key_level = leaf_level > key_level ? deepest : leaf_level;
+    }
+    const int depth = leaf_level + 1;
+    T.depth = depth;
+    std::copy(info->geom, info->geom + 4, T.geom_host);
     T.cnt.assign(depth, 0);
     T.lkeys.assign(depth, nullptr);
     T.lbegin.assign(depth, nullptr);
     T.lut.assign(depth, nullptr);
-    uint32_t* flags_ws = take<uint32_t>(A, n);
-    uint32_t* excl_ws = take<uint32_t>(A, n);
-    uint32_t* scan_ws = take<uint32_t>(A, scan_ws_elems(n));
-    T.leaf_of = take<int32_t>(A, n);
-    if (!flags_ws || !excl_ws || !scan_ws || !T.leaf_of) return LFMM_ERR_NOMEM;
-    // Level sizes stay on the device while the levels are compacted: the leaf
-    // level's count is read back once (it bounds the launches above it), then
-    // every coarser level is sized by the bound min(boxes below, 2^(dim l)),
-    // and all counts and the largest leaf come back in one read.
-    uint32_t* cnt_dev = take<uint32_t>(A, depth);
-    if (!cnt_dev) return LFMM_ERR_NOMEM;
-    LFMM_HIP(hipMemsetAsync(cnt_dev, 0, sizeof(uint32_t) * depth, st));
-    {
-        const int64_t cap = std::min<int64_t>(n, (int64_t)1 << std::min(60, dim * leaf_level));
-        T.lkeys[leaf_level] = take<uint64_t>(A, cap);
-        T.lbegin[leaf_level] = take<int32_t>(A, cap + 1);
-        if (!T.lkeys[leaf_level] || !T.lbegin[leaf_level]) return LFMM_ERR_NOMEM;
-        LFMM_HIP(run_compact(skeys, n, 0, flags_ws, excl_ws, scan_ws, T.lkeys[leaf_level], T.lbegin[leaf_level],
-                             T.leaf_of, &T.cnt[leaf_level], st));
+    int64_t total = 0, dense = 0;
+    LevelOut lv{};
+    for (int l = 0; l < depth; ++l) {
+        T.cnt[l] = lv.count[l] = info->count[l];
+        total += T.cnt[l];
+        if (!keep_parents && l >= 2 && l <= lut_max_level(dim)) dense += (int64_t)1 << (dim * l);
     }
-    if (keep_parents) T.uparent.assign(depth, nullptr);
-    std::vector<int64_t> bound(depth, 0);
-    bound[leaf_level] = T.cnt[leaf_level];
-    for (int l = leaf_level - 1; l >= 0; --l) {
-        const int64_t m = bound[l + 1];
-        bound[l] = std::min<int64_t>(m, (int64_t)1 << (dim * l));
-        T.lkeys[l] = take<uint64_t>(A, bound[l]);
-        T.lbegin[l] = take<int32_t>(A, bound[l] + 1);
-        if (!T.lkeys[l] || !T.lbegin[l]) return LFMM_ERR_NOMEM;
+    uint64_t* akeys = take<uint64_t>(A, total);
+    int32_t* abegin = take<int32_t>(A, total + depth);
+    int32_t* alut = dense > 0 ? take<int32_t>(A, dense) : nullptr;
+    int32_t *afirst = nullptr, *aparent = nullptr;
+    if (!akeys || !abegin || (dense > 0 && !alut)) return LFMM_ERR_NOMEM;
+    if (keep_parents) {
+        afirst = take<int32_t>(A, total + depth);
+        aparent = take<int32_t>(A, total);
+        if (!afirst || !aparent) return LFMM_ERR_NOMEM;
+        T.ufirst.assign(depth, nullptr);
+        T.uparent.assign(depth, nullptr);
+    }
+    if (dense > 0) LFMM_HIP(fill_u32((uint32_t*)alut, dense, 0xffffffffu, st));
+    for (int l = 0; l < depth; ++l) {
+        lv.keys[l] = T.lkeys[l] = akeys;
+        lv.begin[l] = T.lbegin[l] = abegin;
+        akeys += T.cnt[l];
+        abegin += T.cnt[l] + 1;
         if (keep_parents) {
-            T.uparent[l + 1] = take<int32_t>(A, m);
-            if (!T.uparent[l + 1]) return LFMM_ERR_NOMEM;
+            lv.first[l] = T.ufirst[l] = afirst;
+            lv.parent[l] = l > 0 ? aparent : nullptr;
+            T.uparent[l] = aparent;
+            afirst += T.cnt[l] + 1;
+            aparent += T.cnt[l];
+        } else if (l >= 2 && l <= lut_max_level(dim)) {
+            lv.lut[l] = T.lut[l] = alut;
+            alut += (int64_t)1 << (dim * l);
         }
-        LFMM_HIP(run_compact_dev(T.lkeys[l + 1], m, l + 1 == leaf_level ? nullptr : cnt_dev + l + 1, dim, flags_ws,
-                                 excl_ws, scan_ws, T.lkeys[l], T.lbegin[l], keep_parents ? T.uparent[l + 1] : nullptr,
-                                 cnt_dev + l, st));
     }
-    LFMM_HIP(max_run(T.lbegin[leaf_level], T.cnt[leaf_level], umax, nullptr, st));
-    {
-        std::vector<uint32_t> h(depth);
-        LFMM_HIP(hipMemcpyAsync(h.data(), cnt_dev, sizeof(uint32_t) * depth, hipMemcpyDeviceToHost, st));
-        LFMM_HIP(hipMemcpyAsync(&T.max_leaf, umax, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        LFMM_HIP(hipMemcpyAsync(T.geom_host, geom, 4 * sizeof(double), hipMemcpyDeviceToHost, st));
-        LFMM_HIP(hipStreamSynchronize(st));
-        for (int l = 0; l < leaf_level; ++l) T.cnt[l] = h[l];
+    lv.leaf_of = T.leaf_of;
+    LFMM_HIP(emit_levels(dim, skeys, n, key_level, leaf_level, sums, lv, st));
+    if (leaf_level < key_level) {
+        uint32_t* sorted = take<uint32_t>(A, n);
+        if (!sorted) return LFMM_ERR_NOMEM;
+        LFMM_HIP(leaf_order(T.leaf_of, T.lbegin[leaf_level], n, order, sorted, st));
+        order = sorted;
     }
+    T.order = order;
     if (dq) {
         // q != 0 first inside every leaf, then the sorted sources
         if (partition) LFMM_HIP(partition_leaves(T.lbegin[leaf_level], T.cnt[leaf_level], order, dq, qs, st));
         T.src = take<double4>(A, n);
         if (!T.src) return LFMM_ERR_NOMEM;
         LFMM_HIP(gather_sources(dim, dpos, ps, dq, qs, order, n, T.src, st));
-    }
-    for (int l = 2; l < depth; ++l) {
-        if (l > lut_max_level(dim)) continue;
-        T.lut[l] = take<int32_t>(A, (int64_t)1 << (dim * l));
-        if (!T.lut[l]) return LFMM_ERR_NOMEM;
-        LFMM_HIP(build_lut(dim, T.lkeys[l], T.cnt[l], l, T.lut[l], st));
     }
     return LFMM_OK;
 }
@@ -451,7 +436,6 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
     if (adaptive) {
         rc = build_adaptive(ctx, leaf_max, T, fs ? fs->level : 0);
         if (rc != LFMM_OK) return rc;
-        LFMM_HIP(max_run(T.leaf_begin, T.nleaf, T.umax, &T.max_leaf, st));
     }
     const int depth = T.depth;
     const int leaf_level = depth - 1;
@@ -485,10 +469,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
     BoxOrders O;
     if (adaptive && !per_box && N >= 1 && N <= LFMM_MAX_TERMS_3D) {
         // one order: the buckets are the parent lists of the levels
-        uint32_t* leaf_terms = take<uint32_t>(A, T.nleaf);
-        if (!leaf_terms) return LFMM_ERR_NOMEM;
-        LFMM_HIP(fill_u32(leaf_terms, T.nleaf, (uint32_t)N, st));
-        if ((rc = order_box_terms(ctx, T, leaf_terms, mfl, O)) != LFMM_OK) return rc;
+        if ((rc = order_class_lists(ctx, T, N, mfl, O)) != LFMM_OK) return rc;
     }
     if (per_box) {
         const DevTables* DTf = nullptr;  // direction tables (the same for every N)
@@ -920,6 +901,8 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
         la.local = inner_all;
         la.nbr = T.n_rng;
         la.nbr_off = T.n_off;
+        la.near_total = T.n_sources;
+        la.near_runs = T.n_runs;
         la.box_range = T.range_all;
         la.direct_max = kDirectMax;
         la.leaf_lvl = T.leaf_lvl;
@@ -939,9 +922,14 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
         }
     } else {
         int2* nbr = take<int2>(A, cnt[leaf_level] * 27);
-        if (!nbr) return LFMM_ERR_NOMEM;
-        LFMM_HIP(launch_leaf_ranges(lkeys[leaf_level], lbegin[leaf_level], (int)cnt[leaf_level], leaf_level, la.lut, nbr, st));
+        int32_t* total = take<int32_t>(A, cnt[leaf_level]);
+        int32_t* runs = take<int32_t>(A, cnt[leaf_level]);
+        if (!nbr || !total || !runs) return LFMM_ERR_NOMEM;
+        LFMM_HIP(launch_leaf_ranges(lkeys[leaf_level], lbegin[leaf_level], (int)cnt[leaf_level], leaf_level, la.lut, nbr,
+                                    total, runs, st));
         la.nbr = nbr;
+        la.near_total = total;
+        la.near_runs = runs;
     }
     la.n = n;
     la.n_out = n_out;
@@ -1263,6 +1251,11 @@ int lfmm_create(lfmm_ctx** out, int device)
         return LFMM_ERR_HIP;
     }
     c->stream = c->own_stream;
+    if (hipHostMalloc(&c->host_info, kHostInfoBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipStreamDestroy(c->own_stream);
+        delete c;
+        return LFMM_ERR_HIP;
+    }
     *out = c;
     return LFMM_OK;
 }
@@ -1281,6 +1274,7 @@ void lfmm_destroy(lfmm_ctx* c)
     free_tables2d(c);
     (void)hipFree(c->vec_tmp);
     (void)hipFree(c->forest_buf);
+    (void)hipHostFree(c->host_info);
     if (c->switch_event) (void)hipEventDestroy(c->switch_event);
     for (auto e : c->events) (void)hipEventDestroy(e);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);

@@ -117,6 +117,7 @@ struct lfmm_ctx {
     size_t forest_bytes = 0;
     hipStream_t side_stream = nullptr;  // the sampled check's direct sums, beside the solve
     hipEvent_t side_events[2] = {nullptr, nullptr};
+    void* host_info = nullptr;          // kHostInfoBytes of pinned memory: what tree kernels report to the host
     std::mutex mu;
 };
 
@@ -155,7 +156,8 @@ struct Tree {
     std::vector<int32_t*> lut;
     uint32_t max_leaf = 0;
     // uniform build with keep_parents: parent index of every box at levels >= 1
-    std::vector<int32_t*> uparent;
+    // (no lut then), and the first particle of every box
+    std::vector<int32_t*> uparent, ufirst;
     // ---- adaptive octree (build_adaptive).  cnt / lkeys / lbegin / lut then
     // describe the kept boxes of each level (lbegin: child ranges, empty for
     // a leaf); boxes are also numbered globally (gid), level by level.
@@ -181,6 +183,8 @@ struct Tree {
     int32_t* w_gid = nullptr;         //   boxes whose multipoles act on the leaf
     uint32_t* n_off = nullptr;        // near lists of the pair kernel: [nleaf + 1] offsets into n_rng
     int2* n_rng = nullptr;            //   U, the leaf's X sources, W boxes of <= kDirectMax particles
+    int32_t* n_sources = nullptr;     //   [nleaf] particles in the list, and its ranges
+    int32_t* n_runs = nullptr;
     int64_t n_total = 0;
     int total() const { return loff.empty() ? 0 : loff.back(); }
     AdLevels view() const;
@@ -264,6 +268,8 @@ int order_leaf_terms_from_requests(hipStream_t st, const Tree& T, const int32_t*
                                    uint32_t* leaf_terms);
 // Box terms and the (level, terms) launch buckets of the boxes of levels >= first_bucket_level.  promote:
 // buckets of few boxes take the next larger order of their level (fewer launches).  Synchronises.
+// The same for one order everywhere: plist and seg by class alone.
+int order_class_lists(lfmm_ctx* ctx, const Tree& T, int terms, int first_bucket_level, BoxOrders& O);
 int order_box_terms(lfmm_ctx* ctx, const Tree& T, const uint32_t* leaf_terms, int first_bucket_level, BoxOrders& O,
                     bool promote = false);
 // Algorithmic FP64 flops of all M2L operations at their orders (levels below

@@ -39,47 +39,18 @@ __device__ __forceinline__ double rsqrt_nf(double r2)
     return y * fma(-hr * y, y, 1.5);
 }
 
-// Near-source ranges of a leaf: 27 per leaf (uniform tree), or the CSR U list
-// of the adaptive tree (nbr_off).
-__device__ inline void leaf_ranges(const int2* nbr, const uint32_t* nbr_off, int leaf, const int2*& nr, int& cnt)
-{
-    if (nbr_off) {
-        const uint32_t b = nbr_off[leaf];
-        nr = nbr + b;
-        cnt = (int)(nbr_off[leaf + 1] - b);
-    } else {
-        nr = nbr + (int64_t)leaf * 27;
-        cnt = 27;
-    }
-}
-
-// total[leaf]: sources in its near ranges; runs[leaf]: its non-empty near
-// ranges (the uniform table ends with empty ones).  Every WIDTH leaves are
-// ordered by their total, so that the leaves of a wave end together: leaf l is
-// pos[l] in lane order, cnt[pos]: its lanes.
+// Every WIDTH leaves are ordered by the sources of their near lists, so that
+// the leaves of a wave end together: leaf l is pos[l] in lane order,
+// cnt[pos]: its lanes.
 template <int TPL, int WIDTH>
-__global__ void __launch_bounds__(512) k_pair_counts(const int32_t* __restrict__ leaf_begin, const int2* __restrict__ nbr,
-                                                    const uint32_t* __restrict__ nbr_off, int nleaf,
-                                                    uint32_t* __restrict__ cnt, int32_t* __restrict__ pos,
-                                                    int32_t* __restrict__ total, int32_t* __restrict__ runs)
+__global__ void __launch_bounds__(512) k_pair_counts(const int32_t* __restrict__ leaf_begin,
+                                                    const int32_t* __restrict__ near_total, int nleaf,
+                                                    uint32_t* __restrict__ cnt, int32_t* __restrict__ pos)
 {
     __shared__ uint64_t key[512];
     const int base = blockIdx.x * blockDim.x, l = base + threadIdx.x;
-    uint64_t mine = ~0ull;  // past the last leaf: sorts last
-    if (l < nleaf) {
-        const int2* nr;
-        int nc;
-        leaf_ranges(nbr, nbr_off, l, nr, nc);
-        int t = 0, k = 0;
-        for (; k < nc; ++k) {
-            const int2 r = nr[k];
-            if (r.y <= r.x) break;
-            t += r.y - r.x;
-        }
-        total[l] = t;
-        runs[l] = k;
-        mine = ((uint64_t)(uint32_t)t << 32) | threadIdx.x;
-    }
+    // past the last leaf: sorts last
+    const uint64_t mine = l < nleaf ? ((uint64_t)(uint32_t)near_total[l] << 32) | threadIdx.x : ~0ull;
     int leaf = l;
     if constexpr (WIDTH > 1) {  // bitonic
         key[threadIdx.x] = mine;
@@ -155,8 +126,7 @@ __device__ __forceinline__ void p2p_write(const LeafArgs& a, int64_t s, double q
 template <int TPL>
 __global__ void __launch_bounds__(256) k_p2p_multi(LeafArgs a, const int32_t* __restrict__ lanes,
                                                   const uint32_t* __restrict__ slot_begin,
-                                                  const uint32_t* __restrict__ cnt, const int32_t* __restrict__ near_total,
-                                                  const int32_t* __restrict__ near_runs, int parts,
+                                                  const uint32_t* __restrict__ cnt, int parts,
                                                   double4* __restrict__ part_out)
 {
     const int blk = xcd_local_block(blockIdx.x, gridDim.x);
@@ -184,14 +154,13 @@ __global__ void __launch_bounds__(256) k_p2p_multi(LeafArgs a, const int32_t* __
             fz[u] = f.w;
         }
     }
-    const int2* nr;
-    int nrc;
-    leaf_ranges(a.nbr, a.nbr_off, leaf, nr, nrc);
-    nrc = active ? near_runs[leaf] : 0;
+    // near-source ranges: 27 entries per leaf (uniform tree) or a CSR list
+    const int2* nr = a.nbr + (a.nbr_off ? (int64_t)a.nbr_off[leaf] : (int64_t)leaf * 27);
+    const int nrc = active ? a.near_runs[leaf] : 0;
     const double sc = a.leaf_scale ? a.leaf_scale[leaf] : 1.0;
     const double r2min = 1.e-8 * (sc * sc);  // (1e-4 in the system's units)^2
     // this part of the list: its first source's range and offset there
-    const int all = active ? near_total[leaf] : 0;
+    const int all = active ? a.near_total[leaf] : 0;
     const int first = (int)((int64_t)all * part / parts);
     int nsrc = (int)((int64_t)all * (part + 1) / parts) - first;
     const int left = nsrc;
@@ -301,7 +270,7 @@ static int p2p_parts(int64_t n, int64_t nleaf)
     return (int)std::max<int64_t>(1, std::min<int64_t>({16384 / waves, near / 128, 64}));
 }
 
-static int64_t p2p_head_elems(int64_t n, int64_t nleaf) { return (lane_bound(n, nleaf, 2) + 5 * nleaf + 7) / 8 * 8; }
+static int64_t p2p_head_elems(int64_t n, int64_t nleaf) { return (lane_bound(n, nleaf, 2) + 3 * nleaf + 7) / 8 * 8; }
 
 int64_t p2p_ws_elems(int64_t n, int64_t nleaf)
 {
@@ -312,12 +281,10 @@ int64_t p2p_ws_elems(int64_t n, int64_t nleaf)
 template <int TPL>
 static hipError_t p2p_launch(const LeafArgs& a, int32_t* ws, uint32_t* scan_ws, hipStream_t st)
 {
-    // ws: cnt, slot_begin, total, runs, pos [nleaf each], lanes [lane_bound], then the parts' sums
+    // ws: cnt, slot_begin, pos [nleaf each], lanes [lane_bound], then the parts' sums
     uint32_t* cnt = (uint32_t*)ws;
     uint32_t* slot = cnt + a.nleaf;
-    int32_t* total = (int32_t*)(slot + a.nleaf);
-    int32_t* runs = total + a.nleaf;
-    int32_t* pos = runs + a.nleaf;
+    int32_t* pos = (int32_t*)(slot + a.nleaf);
     int32_t* lanes = pos + a.nleaf;
     const int parts = p2p_parts(a.n, a.nleaf);
     double4* part_out = parts > 1 ? (double4*)(ws + p2p_head_elems(a.n, a.nleaf)) : nullptr;
@@ -329,20 +296,20 @@ static hipError_t p2p_launch(const LeafArgs& a, int32_t* ws, uint32_t* scan_ws, 
     // unordered, 4.9 with 32, 6.2 with 256), or none (64 leaves).
     const dim3 grid(nblk(a.nleaf, 512)), block(512);
     if (a.nbr_off)
-        hipLaunchKernelGGL((k_pair_counts<TPL, 512>), grid, block, 0, st, a.leaf_begin, a.nbr, a.nbr_off, a.nleaf, cnt, pos, total, runs);
+        hipLaunchKernelGGL((k_pair_counts<TPL, 512>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos);
     else if (a.nleaf >= 2048)
-        hipLaunchKernelGGL((k_pair_counts<TPL, 256>), grid, block, 0, st, a.leaf_begin, a.nbr, a.nbr_off, a.nleaf, cnt, pos, total, runs);
+        hipLaunchKernelGGL((k_pair_counts<TPL, 256>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos);
     else if (a.nleaf >= 256)
-        hipLaunchKernelGGL((k_pair_counts<TPL, 32>), grid, block, 0, st, a.leaf_begin, a.nbr, a.nbr_off, a.nleaf, cnt, pos, total, runs);
+        hipLaunchKernelGGL((k_pair_counts<TPL, 32>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos);
     else
-        hipLaunchKernelGGL((k_pair_counts<TPL, 1>), grid, block, 0, st, a.leaf_begin, a.nbr, a.nbr_off, a.nleaf, cnt, pos, total, runs);
+        hipLaunchKernelGGL((k_pair_counts<TPL, 1>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos);
     hipError_t e = exclusive_scan(cnt, slot, a.nleaf, scan_ws, st);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((k_pair_lanes<TPL>), dim3(nblk(a.n, 256)), dim3(256), 0, st, a.leaf_of, a.leaf_begin, pos, slot,
                        a.n, lanes);
     const int64_t bound = lane_bound(a.n, a.nleaf, TPL);
-    hipLaunchKernelGGL((k_p2p_multi<TPL>), dim3(nblk(bound, 256) * parts), dim3(256), 0, st, a, lanes, slot, cnt, total,
-                       runs, parts, part_out);
+    hipLaunchKernelGGL((k_p2p_multi<TPL>), dim3(nblk(bound, 256) * parts), dim3(256), 0, st, a, lanes, slot, cnt, parts,
+                       part_out);
     if (parts > 1) hipLaunchKernelGGL(k_p2p_join, dim3(nblk(a.n, 256)), dim3(256), 0, st, a, part_out, parts);
     return hipGetLastError();
 }

@@ -7,18 +7,40 @@
 
 namespace lfmm {
 
+constexpr int kMaxLevels = 32;
+constexpr int kHostInfoBytes = 4096;  // pinned host memory that build kernels write for the host
+
+// What the host reads of a build: level sizes, the fullest boxes and the
+// level that fits leaf_max (see count_levels), geom[0..4].
+struct LevelInfo {
+    uint32_t count[kMaxLevels];
+    uint32_t most[3];
+    double geom[5];
+};
+
+// Level arrays (l <= leaf level): keys and begin have count[l] (+ 1) entries;
+// begin: first child, at the leaves first particle; optional: first = first
+// particle, parent = box number one level up, lut = dense key -> box (holds -1
+// everywhere).  leaf_of[particle] = its leaf.
+struct LevelOut {
+    uint64_t* keys[kMaxLevels];
+    int32_t* begin[kMaxLevels];
+    int32_t* first[kMaxLevels];
+    int32_t* parent[kMaxLevels];
+    int32_t* lut[kMaxLevels];
+    uint32_t count[kMaxLevels];
+    int32_t* leaf_of;
+};
+
 // dim = 2 (quadtree, x << 1 | y keys) or 3 (octree).
-// geom[4] = {shift_x, shift_y, shift_z, scale}; part needs 6 * 1024 doubles.
-hipError_t extent(int dim, const double* pos, int64_t stride, int64_t n, double* part, int* nonfinite, double* geom,
-                  hipStream_t st);
+// geom[5] = {shift_x, shift_y, shift_z, scale, 1 if a coordinate is not finite};
+// part needs 7 * 1024 doubles.
+hipError_t extent(int dim, const double* pos, int64_t stride, int64_t n, double* part, double* geom, hipStream_t st);
+// v: 0 .. n - 1; clear[0 .. 2] = 0
 hipError_t keys(int dim, const double* pos, int64_t stride, int64_t n, int bits, const double* geom, uint64_t* k,
-                uint32_t* v, hipStream_t st);
-// counts_ws: sum_{l<=max_level} 2^(dim l) uint32; maxv_ws: max_level+1 uint32.  Synchronises.
-// *level_out = the smallest level <= max_level whose fullest box holds at
-// most leaf_max particles, or max_level + 1 if there is none.
-hipError_t occupancy_depth(int dim, const double* pos, int64_t stride, int64_t n, const double* geom, int leaf_max,
-                           int max_level, uint32_t* counts_ws, uint32_t* maxv_ws, int* level_out, hipStream_t st);
+                uint32_t* v, uint32_t* clear, hipStream_t st);
 int64_t scan_ws_elems(int64_t n);
+// out[j] = in[0] + .. + in[j - 1]; ws: scan_ws_elems(n).  May be in place.
 hipError_t exclusive_scan(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* ws, hipStream_t st);
 int64_t sort_ws_bytes(int64_t n);
 // Stable LSD radix sort of (keys, vals) on the low `bits` bits; results land
@@ -33,10 +55,21 @@ hipError_t partition_leaves(const int32_t* begin, int64_t nleaf, uint32_t* order
                             hipStream_t st);
 hipError_t gather_sources(int dim, const double* pos, int64_t pstride, const double* q, int64_t qstride,
                           const uint32_t* order, int64_t n, double4* src, hipStream_t st);
-// Run-length compaction of sorted keys at shift sh.  Synchronises (reads the count).
-hipError_t run_compact(const uint64_t* keys, int64_t m, int sh, uint32_t* flags, uint32_t* excl, uint32_t* scan_ws,
-                       uint64_t* ukeys, int32_t* begin, int32_t* owner, int64_t* count_out, hipStream_t st);
-hipError_t build_lut(int dim, const uint64_t* ukeys, int64_t count, int level, int32_t* lut, hipStream_t st);
+// Levels of sorted keys of level key_level.  count_levels: sizes to *host
+// (pinned; there once the stream is waited for), with the fullest box of
+// key_level and of the level above (most[0], most[1]) and, for leaf_max > 0, the
+// smallest level at which no box holds more than leaf_max particles (most[2];
+// key_level + 1: none); most: 3 words, 0 before; sums [level_tiles(n) *
+// (key_level + 1)].  emit_levels then fills the arrays of levels 0 ..
+// leaf_level <= key_level, and leaf_order puts the particles of every leaf
+// back in input order (needed where leaf_level < key_level).
+int64_t level_tiles(int64_t n);
+hipError_t count_levels(int dim, const uint64_t* keys, int64_t n, int key_level, int leaf_max, uint32_t* sums,
+                        const double* geom, uint32_t* most, LevelInfo* host, hipStream_t st);
+hipError_t emit_levels(int dim, const uint64_t* keys, int64_t n, int key_level, int leaf_level, const uint32_t* sums,
+                       const LevelOut& out, hipStream_t st);
+hipError_t leaf_order(const int32_t* leaf_of, const int32_t* begin, int64_t n, const uint32_t* in, uint32_t* out,
+                      hipStream_t st);
 // Exact M2L and near-field pair counts of a built tree (report only); ws
 // holds 2 + depth counters, m2l_per_level (optional) depth entries;
 // p2p_reads (optional): the particles of every leaf's near list, summed over
@@ -47,12 +80,4 @@ hipError_t count_ops(int dim, const std::vector<uint64_t*>& keys, const std::vec
                      int64_t* p2p_reads = nullptr);
 // p[0..n) = v with a fill kernel (safe inside stream capture)
 hipError_t fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t st);
-hipError_t max_run(const int32_t* begin, int64_t count, uint32_t* maxv_dev, uint32_t* out_host, hipStream_t st);
-// run_compact with the counts on the device: at most `bound` elements,
-// *m_dev of them (null: all `bound`); the number of runs goes to *count_dev.
-// No host synchronisation.
-hipError_t run_compact_dev(const uint64_t* keys, int64_t bound, const uint32_t* m_dev, int sh, uint32_t* flags,
-                           uint32_t* excl, uint32_t* scan_ws, uint64_t* ukeys, int32_t* begin, int32_t* owner,
-                           uint32_t* count_dev, hipStream_t st);
-
 }  // namespace lfmm

@@ -5,7 +5,7 @@
 //   box_extent (:218-284)      -> k_extent_partial / k_extent_final (exact min/max)
 //   MortonCode (:84-99)        -> k_keys (bit-identical key)
 //   counting sort (:329-358)   -> stable LSD radix sort of (key, index)
-//   unique_copy + ranges (:364-423) -> flag / scan / compact per level
+//   unique_copy + ranges (:364-423) -> every level from one pass over the sorted keys
 // The reference's threaded counting sort scatters through atomic cursors, so
 // its in-leaf order depends on timing; the stable order produced here is the
 // order of its serial execution.  Near/far lists are not materialised: on a
@@ -13,8 +13,10 @@
 // and the children of the parent's near boxes beyond that (far), found by
 // key lookup in the operator kernels.
 #include "device_common.h"
+#include "scan.h"
 #include "tree.h"
 #include "ops3d.h"
+
 
 namespace lfmm {
 
@@ -22,7 +24,7 @@ namespace lfmm {
 // D = 2 or 3 coordinates per point; unused axes (z in 2D) report 0.
 template <int D>
 __global__ void __launch_bounds__(256) k_extent_partial(const double* __restrict__ pos, int64_t stride, int64_t n,
-                                                        double* __restrict__ part, int* __restrict__ nonfinite)
+                                                        double* __restrict__ part)
 {
     double mn[3] = {INFINITY, INFINITY, D == 3 ? INFINITY : 0.0}, mx[3] = {-INFINITY, -INFINITY, D == 3 ? -INFINITY : 0.0};
     bool bad = false;
@@ -36,8 +38,7 @@ __global__ void __launch_bounds__(256) k_extent_partial(const double* __restrict
     }
     __shared__ double s[6][256];
     for (int a = 0; a < 3; ++a) { s[a][threadIdx.x] = mn[a]; s[3 + a][threadIdx.x] = mx[a]; }
-    if (bad) atomicOr(nonfinite, 1);
-    __syncthreads();
+    const int any = __syncthreads_or(bad ? 1 : 0);
     for (int w = 128; w > 0; w >>= 1) {
         if (threadIdx.x < w)
             for (int a = 0; a < 3; ++a) {
@@ -46,22 +47,28 @@ __global__ void __launch_bounds__(256) k_extent_partial(const double* __restrict
             }
         __syncthreads();
     }
-    if (threadIdx.x < 6) part[blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
+    if (threadIdx.x < 6) part[blockIdx.x * 7 + threadIdx.x] = s[threadIdx.x][0];
+    if (threadIdx.x == 6) part[blockIdx.x * 7 + 6] = any ? 1.0 : 0.0;
 }
 
 // geom = {shift_x, shift_y, shift_z, scale}: shift = min - 1e-7,
-// scale = max extent + 1e-6 (src/cpu/morton_tree.cpp:293-301).
+// scale = max extent + 1e-6 (src/cpu/morton_tree.cpp:293-301); geom[4] = 1
+// when a coordinate is not finite (every key is 0 then, and the host refuses
+// the input at its first read of the build).
 __global__ void __launch_bounds__(256) k_extent_final(const double* __restrict__ part, int nparts, double* __restrict__ geom)
 {
     __shared__ double s[6][256];
     double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int i = threadIdx.x; i < nparts; i += 256)
+    bool bad = false;
+    for (int i = threadIdx.x; i < nparts; i += 256) {
         for (int a = 0; a < 3; ++a) {
-            v[a] = fmin(v[a], part[i * 6 + a]);
-            v[3 + a] = fmax(v[3 + a], part[i * 6 + 3 + a]);
+            v[a] = fmin(v[a], part[i * 7 + a]);
+            v[3 + a] = fmax(v[3 + a], part[i * 7 + 3 + a]);
         }
+        bad |= part[i * 7 + 6] != 0.0;
+    }
     for (int a = 0; a < 6; ++a) s[a][threadIdx.x] = v[a];
-    __syncthreads();
+    const int any = __syncthreads_or(bad ? 1 : 0);
     for (int w = 128; w > 0; w >>= 1) {
         if (threadIdx.x < w)
             for (int a = 0; a < 3; ++a) {
@@ -78,21 +85,24 @@ __global__ void __launch_bounds__(256) k_extent_final(const double* __restrict__
         geom[1] = s[1][0] - 1.e-7;
         geom[2] = s[2][0] - 1.e-7;
         geom[3] = dw + 1.e-6;
+        geom[4] = any ? 1.0 : 0.0;
     }
 }
 
 // ------------------------------------------------------------------ keys
 // ExpandBits<3>: floor(2^bits * x), x = (p - shift) / scale
-// (src/cpu/morton_tree.cpp:66-82, 93-99).  bits = tree_depth - 1.
+// (src/cpu/morton_tree.cpp:66-82, 93-99).  bits = tree_depth - 1.  Where the
+// extent is so large that its 1e-6 margin is lost, x reaches 1: the last cell.
 __device__ inline uint32_t grid_coord(double p, double shift, double scale, int bits)
 {
     const double x = (p - shift) / scale;
-    return (uint32_t)(uint64_t)((double)(1ull << bits) * x);
+    return min((uint32_t)(uint64_t)((double)(1ull << bits) * x), (1u << bits) - 1u);
 }
 
 template <int D>
 __device__ inline uint64_t point_key(const double* p, const double* geom, int bits)
 {
+    if (geom[4] != 0.0) return 0;
     const uint32_t ix = grid_coord(p[0], geom[0], geom[3], bits);
     const uint32_t iy = grid_coord(p[1], geom[1], geom[3], bits);
     if constexpr (D == 2) return morton2(ix, iy);
@@ -102,157 +112,13 @@ __device__ inline uint64_t point_key(const double* p, const double* geom, int bi
 template <int D>
 __global__ void __launch_bounds__(256) k_keys(const double* __restrict__ pos, int64_t stride, int64_t n, int bits,
                                               const double* __restrict__ geom, uint64_t* __restrict__ keys,
-                                              uint32_t* __restrict__ vals)
+                                              uint32_t* __restrict__ vals, uint32_t* __restrict__ clear)
 {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i < 3) clear[i] = 0u;
     if (i >= n) return;
     keys[i] = point_key<D>(pos + i * stride, geom, bits);
     vals[i] = (uint32_t)i;
-}
-
-// Occupancy histogram at a fixed fine level (used to choose the depth from a
-// leaf-size bound): counts[key] += 1.
-template <int D>
-__global__ void __launch_bounds__(256) k_occupancy(const double* __restrict__ pos, int64_t stride, int64_t n, int bits,
-                                                   const double* __restrict__ geom, uint32_t* __restrict__ counts)
-{
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    atomicAdd(&counts[point_key<D>(pos + i * stride, geom, bits)], 1u);
-}
-
-// counts at level l-1 from level l (2^D children each) and the level maximum.
-template <int D>
-__global__ void __launch_bounds__(256) k_occupancy_up(const uint32_t* __restrict__ fine, int64_t ncoarse,
-                                                      uint32_t* __restrict__ coarse, uint32_t* __restrict__ maxv)
-{
-    uint32_t m = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < ncoarse; i += (int64_t)gridDim.x * blockDim.x) {
-        uint32_t s = 0;
-        for (int c = 0; c < (1 << D); ++c) s += fine[i * (1 << D) + c];
-        coarse[i] = s;
-        m = max(m, s);
-    }
-    block_max_u32(m, maxv);
-}
-
-__global__ void __launch_bounds__(256) k_max_u32(const uint32_t* __restrict__ v, int64_t n, uint32_t* __restrict__ maxv)
-{
-    uint32_t m = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        m = max(m, v[i]);
-    block_max_u32(m, maxv);
-}
-
-// ------------------------------------------------------------------ scan
-constexpr int kScanThreads = 256;
-constexpr int kScanItems = 16;
-constexpr int kScanTile = kScanThreads * kScanItems;
-
-__device__ inline uint32_t wave_incl_scan(uint32_t v)
-{
-    const int lane = threadIdx.x & 63;
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t t = (uint32_t)__shfl_up((int)v, off);
-        if (lane >= off) v += t;
-    }
-    return v;
-}
-
-// Block-wide exclusive scan of one value per thread; returns the block total.
-__device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t& total)
-{
-    __shared__ uint32_t wsum[kScanThreads / 64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t inc = wave_incl_scan(v);
-    if (lane == 63) wsum[w] = inc;
-    __syncthreads();
-    uint32_t off = 0, tot = 0;
-    for (int i = 0; i < kScanThreads / 64; ++i) {
-        if (i < w) off += wsum[i];
-        tot += wsum[i];
-    }
-    __syncthreads();
-    total = tot;
-    return off + inc - v;
-}
-
-__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const uint32_t* __restrict__ in, int64_t n,
-                                                              uint32_t* __restrict__ sums)
-{
-    const int64_t base = blockIdx.x * (int64_t)kScanTile;
-    uint32_t s = 0;
-    for (int i = 0; i < kScanItems; ++i) {
-        const int64_t j = base + i * kScanThreads + threadIdx.x;
-        if (j < n) s += in[j];
-    }
-    for (int off = 32; off > 0; off >>= 1) s += (uint32_t)__shfl_xor((int)s, off);
-    __shared__ uint32_t ws[kScanThreads / 64];
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t t = 0;
-        for (int i = 0; i < kScanThreads / 64; ++i) t += ws[i];
-        sums[blockIdx.x] = t;
-    }
-}
-
-// Single-block exclusive scan of the block sums (nb <= 1024 * 64).
-__global__ void __launch_bounds__(1024) k_scan_top(uint32_t* __restrict__ sums, int nb, uint32_t* __restrict__ total)
-{
-    const int per = (nb + 1023) / 1024;
-    const int b0 = threadIdx.x * per;
-    uint32_t s = 0;
-    for (int i = 0; i < per; ++i)
-        if (b0 + i < nb) s += sums[b0 + i];
-    // block scan over 1024 threads
-    __shared__ uint32_t ws[16];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t inc = wave_incl_scan(s);
-    if (lane == 63) ws[w] = inc;
-    __syncthreads();
-    uint32_t off = 0, tot = 0;
-    for (int i = 0; i < 16; ++i) {
-        if (i < w) off += ws[i];
-        tot += ws[i];
-    }
-    uint32_t run = off + inc - s;
-    for (int i = 0; i < per; ++i)
-        if (b0 + i < nb) {
-            const uint32_t t = sums[b0 + i];
-            sums[b0 + i] = run;
-            run += t;
-        }
-    if (threadIdx.x == 0 && total) *total = tot;
-}
-
-__global__ void __launch_bounds__(kScanThreads) k_scan_down(const uint32_t* __restrict__ in, int64_t n,
-                                                            const uint32_t* __restrict__ sums, uint32_t* __restrict__ out)
-{
-    __shared__ uint32_t tile[kScanTile];
-    const int64_t base = blockIdx.x * (int64_t)kScanTile;
-    for (int i = 0; i < kScanItems; ++i) {
-        const int64_t j = base + i * kScanThreads + threadIdx.x;
-        tile[i * kScanThreads + threadIdx.x] = j < n ? in[j] : 0u;
-    }
-    __syncthreads();
-    uint32_t loc[kScanItems];
-    uint32_t s = 0;
-    for (int i = 0; i < kScanItems; ++i) {
-        loc[i] = tile[threadIdx.x * kScanItems + i];
-        s += loc[i];
-    }
-    uint32_t tot;
-    uint32_t run = block_excl_scan(s, tot) + sums[blockIdx.x];
-    for (int i = 0; i < kScanItems; ++i) {
-        tile[threadIdx.x * kScanItems + i] = run;
-        run += loc[i];
-    }
-    __syncthreads();
-    for (int i = 0; i < kScanItems; ++i) {
-        const int64_t j = base + i * kScanThreads + threadIdx.x;
-        if (j < n) out[j] = tile[i * kScanThreads + threadIdx.x];
-    }
 }
 
 // ------------------------------------------------------------------ radix sort
@@ -388,85 +254,220 @@ __global__ void __launch_bounds__(256) k_gather(const double* __restrict__ pos, 
 }
 
 // ------------------------------------------------------------------ levels
-// flags[i] = 1 where (key[i] >> sh) starts a new run.
-__global__ void __launch_bounds__(256) k_run_flags(const uint64_t* __restrict__ keys, int64_t m, int sh,
-                                                   uint32_t* __restrict__ flags)
+// All levels from one pass over the sorted keys.  A particle whose key differs
+// from the one before it starts a box at the level of the highest digit that
+// differs and at every finer one: a box's number at level l is the count of
+// the starts at l before it.  Three launches (count per tile, scan of the
+// tiles, write) and one read of the level sizes in between; level by level it
+// took five launches each.
+constexpr int kLvItems = 4;
+constexpr int kLvTile = 256 * kLvItems;  // small: 65,536 particles make 64 workgroups
+
+// first level at which a particle of key k (at key_level), the one before it
+// of key p, starts a box; 0xff: none
+template <int D>
+__device__ inline uint32_t start_level(uint64_t k, uint64_t p, bool head, int key_level)
 {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    flags[i] = (i == 0 || (keys[i] >> sh) != (keys[i - 1] >> sh)) ? 1u : 0u;
+    if (head) return 0;
+    const uint64_t x = k ^ p;
+    return x ? (uint32_t)(key_level - (63 - __clzll((long long)x)) / D) : 0xffu;
 }
 
-// Compaction: run r starts at element begin[r] with key (key >> sh);
-// owner[i] = run index of element i.  begin[count] = m.
-__global__ void __launch_bounds__(256) k_run_compact(const uint64_t* __restrict__ keys, int64_t m, int sh,
-                                                     const uint32_t* __restrict__ flags, const uint32_t* __restrict__ excl,
-                                                     uint64_t* __restrict__ ukeys, int32_t* __restrict__ begin,
-                                                     int32_t* __restrict__ owner)
+// sums[l * tiles + t]: boxes of level l that start in tile t.  most[0] and
+// most[1] grow to the fullest box of the keys' level and of the one above;
+// most[2] to the smallest level at which no box holds more than leaf_max
+// (key_level + 1: there is none): keys leaf_max places apart share a box above
+// that level.
+template <int D>
+__global__ void __launch_bounds__(256) k_level_count(const uint64_t* __restrict__ keys, int64_t n, int key_level,
+                                                     int64_t leaf_max, uint32_t* __restrict__ sums,
+                                                     uint32_t* __restrict__ most)
 {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const uint32_t r = excl[i] + flags[i] - 1u;
-    if (flags[i]) {
-        ukeys[r] = keys[i] >> sh;
-        begin[r] = (int32_t)i;
+    constexpr int kWords = kLvTile / 64;
+    __shared__ uint32_t h[kMaxLevels];
+    __shared__ uint64_t starts[2][kWords];  // bit per particle of the tile: starts a box of key_level (- 1)
+    if (threadIdx.x < kMaxLevels) h[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t base = blockIdx.x * (int64_t)kLvTile;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    uint32_t q[kLvItems], need = 0;
+#pragma unroll
+    for (int r = 0; r < kLvItems; ++r) {
+        const int64_t i = base + r * 256 + threadIdx.x;
+        q[r] = i < n ? start_level<D>(keys[i], keys[i > 0 ? i - 1 : 0], i == 0, key_level) : 0xffu;
+        if (leaf_max > 0 && i + leaf_max < n) {
+            const uint32_t d = start_level<D>(keys[i], keys[i + leaf_max], false, key_level);
+            need = max(need, d == 0xffu ? (uint32_t)key_level + 1 : d);
+        }
     }
-    if (owner) owner[i] = (int32_t)r;
-    if (i == m - 1) begin[r + 1] = (int32_t)m;
-}
-
-// The same with the element count on the device (m_dev, at most `bound`
-// elements): the flags and the compaction of a level can follow the previous
-// level's compaction without a host read-back.  *count_dev = runs.
-__global__ void __launch_bounds__(256) k_run_flags_d(const uint64_t* __restrict__ keys, int64_t bound,
-                                                     const uint32_t* __restrict__ m_dev, int sh,
-                                                     uint32_t* __restrict__ flags)
-{
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= bound) return;
-    const int64_t m = m_dev ? (int64_t)*m_dev : bound;
-    flags[i] = (i < m && (i == 0 || (keys[i] >> sh) != (keys[i - 1] >> sh))) ? 1u : 0u;
-}
-
-__global__ void __launch_bounds__(256) k_run_compact_d(const uint64_t* __restrict__ keys, int64_t bound,
-                                                       const uint32_t* __restrict__ m_dev, int sh,
-                                                       const uint32_t* __restrict__ flags,
-                                                       const uint32_t* __restrict__ excl, uint64_t* __restrict__ ukeys,
-                                                       int32_t* __restrict__ begin, int32_t* __restrict__ owner,
-                                                       uint32_t* __restrict__ count_dev)
-{
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int64_t m = m_dev ? (int64_t)*m_dev : bound;
-    if (i >= bound || i >= m) return;
-    const uint32_t r = excl[i] + flags[i] - 1u;
-    if (flags[i]) {
-        ukeys[r] = keys[i] >> sh;
-        begin[r] = (int32_t)i;
+#pragma unroll
+    for (int r = 0; r < kLvItems; ++r) {
+        const uint64_t m0 = __ballot(q[r] != 0xffu), m1 = __ballot((int)q[r] < key_level);
+        if (lane == 0) {
+            starts[0][r * 4 + w] = m0;
+            starts[1][r * 4 + w] = m1;
+        }
+        if (q[r] != 0xffu) atomicAdd(&h[q[r]], 1u);
     }
-    if (owner) owner[i] = (int32_t)r;
-    if (i == m - 1) {
-        begin[r + 1] = (int32_t)m;
-        *count_dev = r + 1;
+    __syncthreads();
+    // a box of level key_level - up ends at the tile's next start
+    auto box_size = [&](int up, int r) -> uint32_t {
+        int word = r * 4 + w;
+        uint64_t m = starts[up][word] & (~0ull << lane << 1);
+        while (m == 0 && ++word < kWords) m = starts[up][word];
+        const int at = r * 256 + threadIdx.x;
+        if (m != 0) return (uint32_t)(word * 64 + __ffsll((unsigned long long)m) - 1 - at);
+        // the tile's last: first place past the tile with another key
+        const int64_t i = base + at;
+        const int sh = D * up;
+        const uint64_t k = keys[i] >> sh;
+        int64_t lo = min(base + kLvTile, n) - 1, step = 1;  // keys[lo] is of the box
+        while (lo + step < n && keys[lo + step] >> sh == k) {
+            lo += step;
+            step *= 2;
+        }
+        int64_t hi = min(lo + step, n);  // keys[hi] is not, or the end
+        while (hi - lo > 1) {
+            const int64_t mid = (lo + hi) / 2;
+            if (keys[mid] >> sh == k) lo = mid;
+            else hi = mid;
+        }
+        return (uint32_t)(hi - i);
+    };
+    uint32_t most0 = 0, most1 = 0;
+#pragma unroll
+    for (int r = 0; r < kLvItems; ++r) {
+        if (q[r] != 0xffu) most0 = max(most0, box_size(0, r));
+        if ((int)q[r] < key_level) most1 = max(most1, box_size(1, r));
+    }
+    block_max_u32(most0, most);
+    __syncthreads();
+    block_max_u32(most1, most + 1);
+    __syncthreads();
+    block_max_u32(need, most + 2);
+    if ((int)threadIdx.x <= key_level) {
+        uint32_t s = 0;
+        for (int l = 0; l <= (int)threadIdx.x; ++l) s += h[l];
+        sums[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
     }
 }
 
-__global__ void __launch_bounds__(256) k_lut_fill(const uint64_t* __restrict__ ukeys, int64_t count, int32_t* __restrict__ lut)
+// One workgroup per level: its tiles' sums become the boxes before the tile,
+// and the host gets the level's size.
+__global__ void __launch_bounds__(1024) k_level_top(uint32_t* __restrict__ sums, int tiles, const double* __restrict__ geom,
+                                                    const uint32_t* __restrict__ most, LevelInfo* __restrict__ host)
 {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i < count) lut[ukeys[i]] = (int32_t)i;
+    uint32_t* v = sums + (int64_t)blockIdx.x * tiles;
+    const int per = (tiles + 1023) / 1024;
+    const int b0 = threadIdx.x * per;
+    uint32_t s = 0;
+    for (int i = 0; i < per; ++i)
+        if (b0 + i < tiles) s += v[b0 + i];
+    uint32_t tot;
+    uint32_t run = block_excl_scan<1024>(s, tot);
+    for (int i = 0; i < per; ++i)
+        if (b0 + i < tiles) {
+            const uint32_t t = v[b0 + i];
+            v[b0 + i] = run;
+            run += t;
+        }
+    if (threadIdx.x == 0) host->count[blockIdx.x] = tot;
+    if (blockIdx.x == 0 && threadIdx.x < 5) host->geom[threadIdx.x] = geom[threadIdx.x];
+    if (blockIdx.x == 0 && threadIdx.x >= 5 && threadIdx.x < 8) host->most[threadIdx.x - 5] = most[threadIdx.x - 5];
+}
+
+// Box numbers of five levels at a time, 12 bits each, in one scan of the tile
+// (it starts at most 1,024 boxes of a level); the coarsest of the five is the
+// finest of the next, since a box needs its parent's and its first child's
+// number.
+template <int D>
+__global__ void __launch_bounds__(256) k_level_emit(const uint64_t* __restrict__ keys, int64_t n, int key_level, int leaf_level,
+                                                    const uint32_t* __restrict__ sums, LevelOut out)
+{
+    constexpr int kBits = 12;
+    constexpr uint64_t kOnes = 0x001001001001001ull, kField = (1u << kBits) - 1;
+    static_assert(kLvTile <= kField, "a field counts a tile");
+    __shared__ uint32_t tile_off[kMaxLevels];
+    const int64_t base = blockIdx.x * (int64_t)kLvTile, i0 = base + threadIdx.x * kLvItems;
+    if ((int)threadIdx.x <= leaf_level) {
+        const int l = threadIdx.x;
+        tile_off[l] = sums[(int64_t)l * gridDim.x + blockIdx.x];
+        if (blockIdx.x == 0) {  // one past the last box
+            out.begin[l][out.count[l]] = l == leaf_level ? (int32_t)n : (int32_t)out.count[l + 1];
+            if (out.first[l]) out.first[l][out.count[l]] = (int32_t)n;
+        }
+    }
+    uint64_t key[kLvItems];
+    int q[kLvItems];
+    uint64_t prev = i0 > 0 && i0 < n ? keys[i0 - 1] : 0;
+#pragma unroll
+    for (int j = 0; j < kLvItems; ++j) key[j] = i0 + j < n ? keys[i0 + j] : 0;
+#pragma unroll
+    for (int j = 0; j < kLvItems; ++j) {
+        q[j] = i0 + j < n ? (int)start_level<D>(key[j], prev, i0 + j == 0, key_level) : 0xff;
+        prev = key[j];
+        key[j] >>= D * (key_level - leaf_level);
+    }
+    __syncthreads();
+    for (int hi = leaf_level;;) {
+        const int lo = max(hi - 4, 0);
+        // a start at level q counts at every level of lo .. hi from q on
+        auto weight = [&](int level) -> uint64_t { return level > hi ? 0ull : kOnes << (kBits * max(level - lo, 0)); };
+        uint64_t s = 0, tot;
+#pragma unroll
+        for (int j = 0; j < kLvItems; ++j) s += weight(q[j]);
+        uint64_t run = block_excl_scan<256>(s, tot);
+#pragma unroll
+        for (int j = 0; j < kLvItems; ++j) {
+            // boxes of level l before particle i0 + j
+            auto before = [&](int l) { return (int32_t)(tile_off[l] + (uint32_t)((run >> (kBits * (l - lo))) & kField)); };
+            if (hi == leaf_level && i0 + j < n) out.leaf_of[i0 + j] = before(hi) + (q[j] <= hi ? 1 : 0) - 1;
+            if (q[j] <= hi) {
+                int32_t b = before(hi);  // of the level below the one at hand, then its own
+                if (hi == leaf_level) {
+                    out.keys[hi][b] = key[j];
+                    out.begin[hi][b] = (int32_t)(i0 + j);
+                    if (out.first[hi]) out.first[hi][b] = (int32_t)(i0 + j);
+                    if (out.lut[hi]) out.lut[hi][key[j]] = b;
+                }
+                for (int l = hi - 1; l >= lo; --l) {
+                    const int32_t u = before(l);
+                    if (out.parent[l + 1]) out.parent[l + 1][b] = u + (q[j] <= l ? 1 : 0) - 1;
+                    if (q[j] > l) break;
+                    const uint64_t k = key[j] >> (D * (leaf_level - l));
+                    out.keys[l][u] = k;
+                    out.begin[l][u] = b;
+                    if (out.first[l]) out.first[l][u] = (int32_t)(i0 + j);
+                    if (out.lut[l]) out.lut[l][k] = u;
+                    b = u;
+                }
+            }
+            run += weight(q[j]);
+        }
+        if (lo == 0) break;
+        hi = lo;
+    }
+}
+
+// Particles of every leaf in input order, where their order came from keys of
+// a finer level: each moves to its rank among its leaf's.  Most of these leaves
+// hold a few particles (7M of them: 0.74 ms with half a wave per leaf).
+__global__ void __launch_bounds__(256) k_leaf_order(const int32_t* __restrict__ leaf_of, const int32_t* __restrict__ begin,
+                                                    int64_t n, const uint32_t* __restrict__ in, uint32_t* __restrict__ out)
+{
+    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    const int leaf = leaf_of[s];
+    const int b = begin[leaf], e = begin[leaf + 1];
+    const uint32_t v = in[s];
+    int at = b;
+    for (int j = b; j < e; ++j) at += in[j] < v ? 1 : 0;
+    out[at] = v;
 }
 
 __global__ void __launch_bounds__(256) k_fill_i32(int32_t* __restrict__ p, int64_t n, int32_t v)
 {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = v;
-}
-
-__global__ void __launch_bounds__(256) k_max_run(const int32_t* __restrict__ begin, int64_t count, uint32_t* __restrict__ maxv)
-{
-    uint32_t m = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
-        m = max(m, (uint32_t)(begin[i + 1] - begin[i]));
-    block_max_u32(m, maxv);
 }
 
 // ------------------------------------------------------------------ counts
@@ -548,11 +549,11 @@ __global__ void __launch_bounds__(256) k_count_p2p(const uint64_t* __restrict__ 
 // Half a wave per leaf: lane o < 27 finds the particle range of neighbour o;
 // the ranges are then put in particle order and runs that touch are joined
 // (Morton order: 27 neighbours make 9 to 10 runs on a full tree), so the pair
-// loop changes ranges a third as often and never meets an empty one.  Unused
-// entries of the leaf's 27 are (0, 0).
+// loop changes ranges a third as often and never meets an empty one.
 __global__ void __launch_bounds__(256) k_leaf_ranges(const uint64_t* __restrict__ leaf_key,
                                                      const int32_t* __restrict__ leaf_begin, int nleaf, int level,
-                                                     const int32_t* __restrict__ lut, int2* __restrict__ nbr)
+                                                     const int32_t* __restrict__ lut, int2* __restrict__ nbr,
+                                                     int32_t* __restrict__ total, int32_t* __restrict__ nruns)
 {
     __shared__ int2 sorted[8][32];
     const int half = threadIdx.x >> 5, o = threadIdx.x & 31;
@@ -583,76 +584,36 @@ __global__ void __launch_bounds__(256) k_leaf_ranges(const uint64_t* __restrict_
     const bool head = ok && (o == 0 || sorted[half][o - 1].y != r.x);
     const bool tail = ok && (o == 31 || sorted[half][o + 1].x != r.y);
     const uint32_t heads = (uint32_t)(__ballot(head) >> (threadIdx.x & 32));
+    int sum = ok ? r.y - r.x : 0;
+    for (int off = 16; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 32);
     if (leaf >= nleaf || o >= 27) return;
     int* out = (int*)(nbr + (int64_t)leaf * 27);
-    const int runs = __popc(heads);
+    if (o == 0) {
+        total[leaf] = sum;
+        nruns[leaf] = __popc(heads);
+    }
     const int run = __popc(heads & ((2u << o) - 1u)) - 1;
     if (head) out[2 * run] = r.x;
     if (tail) out[2 * run + 1] = r.y;
-    if (o >= runs) {
-        out[2 * o] = 0;
-        out[2 * o + 1] = 0;
-    }
 }
 
 // ================================================================== host side
 static inline int nblk(int64_t n, int t) { return (int)((n + t - 1) / t); }
 
-hipError_t extent(int dim, const double* pos, int64_t stride, int64_t n, double* part, int* nonfinite, double* geom,
-                  hipStream_t st)
+hipError_t extent(int dim, const double* pos, int64_t stride, int64_t n, double* part, double* geom, hipStream_t st)
 {
     const int nb = (int)std::min<int64_t>(1024, std::max<int64_t>(1, nblk(n, 256)));
-    if (dim == 2) hipLaunchKernelGGL(k_extent_partial<2>, dim3(nb), dim3(256), 0, st, pos, stride, n, part, nonfinite);
-    else hipLaunchKernelGGL(k_extent_partial<3>, dim3(nb), dim3(256), 0, st, pos, stride, n, part, nonfinite);
+    if (dim == 2) hipLaunchKernelGGL(k_extent_partial<2>, dim3(nb), dim3(256), 0, st, pos, stride, n, part);
+    else hipLaunchKernelGGL(k_extent_partial<3>, dim3(nb), dim3(256), 0, st, pos, stride, n, part);
     hipLaunchKernelGGL(k_extent_final, dim3(1), dim3(256), 0, st, part, nb, geom);
     return hipGetLastError();
 }
 
 hipError_t keys(int dim, const double* pos, int64_t stride, int64_t n, int bits, const double* geom, uint64_t* k,
-                uint32_t* v, hipStream_t st)
+                uint32_t* v, uint32_t* clear, hipStream_t st)
 {
-    if (dim == 2) hipLaunchKernelGGL(k_keys<2>, dim3(nblk(n, 256)), dim3(256), 0, st, pos, stride, n, bits, geom, k, v);
-    else hipLaunchKernelGGL(k_keys<3>, dim3(nblk(n, 256)), dim3(256), 0, st, pos, stride, n, bits, geom, k, v);
-    return hipGetLastError();
-}
-
-hipError_t occupancy_depth(int dim, const double* pos, int64_t stride, int64_t n, const double* geom, int leaf_max,
-                           int max_level, uint32_t* counts_ws, uint32_t* maxv_ws, int* level_out, hipStream_t st)
-{
-    // histogram at max_level, then coarsen level by level; pick the smallest
-    // level whose fullest box holds <= leaf_max particles.
-    const int64_t nb = (int64_t)1 << (dim * max_level);
-    int64_t off = 0;
-    std::vector<int64_t> offs(max_level + 1);
-    for (int l = max_level; l >= 0; --l) { offs[l] = off; off += (int64_t)1 << (dim * l); }
-    hipError_t e = hipMemsetAsync(counts_ws, 0, sizeof(uint32_t) * nb, st);
-    if (e == hipSuccess) e = hipMemsetAsync(maxv_ws, 0, sizeof(uint32_t) * (max_level + 1), st);
-    if (e != hipSuccess) return e;
-    if (dim == 2)
-        hipLaunchKernelGGL(k_occupancy<2>, dim3(nblk(n, 256)), dim3(256), 0, st, pos, stride, n, max_level, geom,
-                           counts_ws + offs[max_level]);
-    else
-        hipLaunchKernelGGL(k_occupancy<3>, dim3(nblk(n, 256)), dim3(256), 0, st, pos, stride, n, max_level, geom,
-                           counts_ws + offs[max_level]);
-    hipLaunchKernelGGL(k_max_u32, dim3((int)std::min<int64_t>(256, nblk(nb, 256))), dim3(256), 0, st,
-                       counts_ws + offs[max_level], nb, maxv_ws + max_level);
-    for (int l = max_level - 1; l >= 0; --l) {
-        const int64_t nc = (int64_t)1 << (dim * l);
-        if (dim == 2)
-            hipLaunchKernelGGL(k_occupancy_up<2>, dim3(std::min(256, nblk(nc, 256))), dim3(256), 0, st, counts_ws + offs[l + 1], nc,
-                               counts_ws + offs[l], maxv_ws + l);
-        else
-            hipLaunchKernelGGL(k_occupancy_up<3>, dim3(std::min(256, nblk(nc, 256))), dim3(256), 0, st, counts_ws + offs[l + 1], nc,
-                               counts_ws + offs[l], maxv_ws + l);
-    }
-    std::vector<uint32_t> mx(max_level + 1);
-    e = hipMemcpyAsync(mx.data(), maxv_ws, sizeof(uint32_t) * (max_level + 1), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) return e;
-    int lvl = max_level + 1;  // none of the dense levels is fine enough
-    for (int l = 0; l <= max_level; ++l)
-        if ((int64_t)mx[l] <= leaf_max) { lvl = l; break; }
-    *level_out = lvl;
+    if (dim == 2) hipLaunchKernelGGL(k_keys<2>, dim3(nblk(n, 256)), dim3(256), 0, st, pos, stride, n, bits, geom, k, v, clear);
+    else hipLaunchKernelGGL(k_keys<3>, dim3(nblk(n, 256)), dim3(256), 0, st, pos, stride, n, bits, geom, k, v, clear);
     return hipGetLastError();
 }
 
@@ -660,12 +621,7 @@ int64_t scan_ws_elems(int64_t n) { return nblk(n, kScanTile) + 1; }
 
 hipError_t exclusive_scan(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* ws, hipStream_t st)
 {
-    const int nb = nblk(n, kScanTile);
-    if (nb > 1024 * 64) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kScanThreads), 0, st, in, n, ws);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, st, ws, nb, ws + nb);
-    hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(kScanThreads), 0, st, in, n, ws, out);
-    return hipGetLastError();
+    return scan_apply(ScanLoad{in}, ScanStore{out}, n, ws, st);
 }
 
 int64_t sort_ws_bytes(int64_t n)
@@ -724,41 +680,34 @@ hipError_t gather_sources(int dim, const double* pos, int64_t pstride, const dou
     return hipGetLastError();
 }
 
-hipError_t run_compact(const uint64_t* keys, int64_t m, int sh, uint32_t* flags, uint32_t* excl, uint32_t* scan_ws,
-                       uint64_t* ukeys, int32_t* begin, int32_t* owner, int64_t* count_out, hipStream_t st)
+int64_t level_tiles(int64_t n) { return nblk(n, kLvTile); }
+
+hipError_t count_levels(int dim, const uint64_t* keys, int64_t n, int key_level, int leaf_max, uint32_t* sums,
+                        const double* geom, uint32_t* most, LevelInfo* host, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_run_flags, dim3(nblk(m, 256)), dim3(256), 0, st, keys, m, sh, flags);
-    hipError_t e = exclusive_scan(flags, excl, m, scan_ws, st);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_run_compact, dim3(nblk(m, 256)), dim3(256), 0, st, keys, m, sh, flags, excl, ukeys, begin, owner);
-    // total = excl[m-1] + flags[m-1]
-    uint32_t tail[2];
-    e = hipMemcpyAsync(&tail[0], excl + (m - 1), 4, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(&tail[1], flags + (m - 1), 4, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) return e;
-    *count_out = (int64_t)tail[0] + tail[1];
+    static_assert(sizeof(LevelInfo) <= kHostInfoBytes, "the host page holds it");
+    const int tiles = (int)level_tiles(n);
+    if (key_level >= kMaxLevels) return hipErrorInvalidValue;
+    const int64_t lm = leaf_max;
+    if (dim == 2) hipLaunchKernelGGL(k_level_count<2>, dim3(tiles), dim3(256), 0, st, keys, n, key_level, lm, sums, most);
+    else hipLaunchKernelGGL(k_level_count<3>, dim3(tiles), dim3(256), 0, st, keys, n, key_level, lm, sums, most);
+    hipLaunchKernelGGL(k_level_top, dim3(key_level + 1), dim3(1024), 0, st, sums, tiles, geom, most, host);
     return hipGetLastError();
 }
 
-hipError_t run_compact_dev(const uint64_t* keys, int64_t bound, const uint32_t* m_dev, int sh, uint32_t* flags,
-                           uint32_t* excl, uint32_t* scan_ws, uint64_t* ukeys, int32_t* begin, int32_t* owner,
-                           uint32_t* count_dev, hipStream_t st)
+hipError_t emit_levels(int dim, const uint64_t* keys, int64_t n, int key_level, int leaf_level, const uint32_t* sums,
+                       const LevelOut& out, hipStream_t st)
 {
-    if (bound <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_run_flags_d, dim3(nblk(bound, 256)), dim3(256), 0, st, keys, bound, m_dev, sh, flags);
-    hipError_t e = exclusive_scan(flags, excl, bound, scan_ws, st);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_run_compact_d, dim3(nblk(bound, 256)), dim3(256), 0, st, keys, bound, m_dev, sh, flags, excl,
-                       ukeys, begin, owner, count_dev);
+    const dim3 grid((unsigned)level_tiles(n)), block(256);
+    if (dim == 2) hipLaunchKernelGGL(k_level_emit<2>, grid, block, 0, st, keys, n, key_level, leaf_level, sums, out);
+    else hipLaunchKernelGGL(k_level_emit<3>, grid, block, 0, st, keys, n, key_level, leaf_level, sums, out);
     return hipGetLastError();
 }
 
-hipError_t build_lut(int dim, const uint64_t* ukeys, int64_t count, int level, int32_t* lut, hipStream_t st)
+hipError_t leaf_order(const int32_t* leaf_of, const int32_t* begin, int64_t n, const uint32_t* in, uint32_t* out,
+                      hipStream_t st)
 {
-    const int64_t span = (int64_t)1 << (dim * level);
-    hipLaunchKernelGGL(k_fill_i32, dim3((int)std::min<int64_t>(4096, nblk(span, 256))), dim3(256), 0, st, lut, span, -1);
-    hipLaunchKernelGGL(k_lut_fill, dim3(nblk(count, 256)), dim3(256), 0, st, ukeys, count, lut);
+    if (n > 0) hipLaunchKernelGGL(k_leaf_order, dim3(nblk(n, 256)), dim3(256), 0, st, leaf_of, begin, n, in, out);
     return hipGetLastError();
 }
 
@@ -800,10 +749,11 @@ hipError_t count_ops(int dim, const std::vector<uint64_t*>& keys, const std::vec
 }
 
 hipError_t launch_leaf_ranges(const uint64_t* leaf_key, const int32_t* leaf_begin, int nleaf, int level,
-                              const int32_t* lut, int2* nbr, hipStream_t st)
+                              const int32_t* lut, int2* nbr, int32_t* total, int32_t* runs, hipStream_t st)
 {
     if (nleaf > 0)
-        hipLaunchKernelGGL(k_leaf_ranges, dim3(nblk(nleaf, 8)), dim3(256), 0, st, leaf_key, leaf_begin, nleaf, level, lut, nbr);
+        hipLaunchKernelGGL(k_leaf_ranges, dim3(nblk(nleaf, 8)), dim3(256), 0, st, leaf_key, leaf_begin, nleaf, level, lut, nbr,
+                           total, runs);
     return hipGetLastError();
 }
 
@@ -813,18 +763,6 @@ hipError_t fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t st)
         hipLaunchKernelGGL(k_fill_i32, dim3((int)std::min<int64_t>(4096, nblk(n, 256))), dim3(256), 0, st, (int32_t*)p, n,
                            (int32_t)v);
     return hipGetLastError();
-}
-
-hipError_t max_run(const int32_t* begin, int64_t count, uint32_t* maxv_dev, uint32_t* out_host, hipStream_t st)
-{
-    hipError_t e = hipMemsetAsync(maxv_dev, 0, 4, st);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_max_run, dim3((int)std::min<int64_t>(256, std::max(1, nblk(count, 256)))), dim3(256), 0, st, begin,
-                       count, maxv_dev);
-    if (!out_host) return hipGetLastError();
-    e = hipMemcpyAsync(out_host, maxv_dev, 4, hipMemcpyDeviceToHost, st);
-    if (e != hipSuccess) return e;
-    return hipStreamSynchronize(st);
 }
 
 }  // namespace lfmm
