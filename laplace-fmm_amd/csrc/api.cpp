@@ -925,7 +925,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
         int32_t* total = take<int32_t>(A, cnt[leaf_level]);
         int32_t* runs = take<int32_t>(A, cnt[leaf_level]);
         if (!nbr || !total || !runs) return LFMM_ERR_NOMEM;
-        LFMM_HIP(launch_leaf_ranges(lkeys[leaf_level], lbegin[leaf_level], (int)cnt[leaf_level], leaf_level, la.lut, nbr,
+        LFMM_HIP(launch_leaf_ranges(3, lkeys[leaf_level], lbegin[leaf_level], (int)cnt[leaf_level], leaf_level, la.lut, nbr,
                                     total, runs, st));
         la.nbr = nbr;
         la.near_total = total;

@@ -1,7 +1,7 @@
 // api2d.cpp -- the 2D (complex-series) FMM through the C ABI: lfmm_fmm2d and
 // lfmm_tree2d.  Same pipeline as the 3D solve on a quadtree:
 //   extent -> keys -> radix sort -> levels -> P2M -> M2M (up)
-//   -> L2L+M2L per level (down) -> L2P+P2P at the leaves, scattered to input order.
+//   -> M2L of all levels, L2L per level (down) -> L2P+P2P at the leaves, scattered to input order.
 // Reference: src/cpu/multipole.cpp (Solve :473-520, parameter rules :478-487).
 #include "api_internal.h"
 #include "ops2d.h"
@@ -28,12 +28,15 @@ static int get_tables2d(lfmm_ctx* ctx, int N, const DevTables2d** out)
     }
     OpTables2d T;
     build_op_tables_2d(N, T);
+    Pack2d K;
+    pack_2d(N, K);
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const std::vector<float> m2l32(T.m2l.begin(), T.m2l.end());  // round to nearest
-    const size_t b1 = T.m2l.size() * 8, b2 = T.m2m.size() * 8, b3 = T.l2l.size() * 8, b4 = T.dir_vec.size() * 4,
-                 b5 = T.class_dirs.size() * 4, b6 = m2l32.size() * 4;
+    std::vector<double> zero(2 * N, 0.0);
+    size_t total = al(T.dir_vec.size() * 4) + al(T.class_dirs.size() * 4) + al(m2l32.size() * 4);
+    for (auto* v : {&K.m2l, &K.src, &K.out, &K.log, &K.m2m, &K.l2l, &K.down, &K.up, &zero}) total += al(v->size() * 8);
     char* blk = nullptr;
-    if (hipMalloc(&blk, al(b1) + al(b2) + al(b3) + al(b4) + al(b5) + al(b6)) != hipSuccess) return LFMM_ERR_NOMEM;
+    if (hipMalloc(&blk, total) != hipSuccess) return LFMM_ERR_NOMEM;
     size_t o = 0;
     bool ok = true;
     auto put = [&](const void* src, size_t bytes) -> void* {
@@ -49,12 +52,18 @@ static int get_tables2d(lfmm_ctx* ctx, int N, const DevTables2d** out)
     }
     D->N = N;
     D->block = blk;
-    D->t.m2l = (const double2*)put(T.m2l.data(), b1);
-    D->t.m2m = (const double2*)put(T.m2m.data(), b2);
-    D->t.l2l = (const double2*)put(T.l2l.data(), b3);
-    D->t.dir_vec = (const int*)put(T.dir_vec.data(), b4);
-    D->t.class_dirs = (const int*)put(T.class_dirs.data(), b5);
-    D->t.m2l32 = (const float2*)put(m2l32.data(), b6);
+    D->t.m2l = (const double*)put(K.m2l.data(), K.m2l.size() * 8);
+    D->t.src = (const double*)put(K.src.data(), K.src.size() * 8);
+    D->t.out = (const double*)put(K.out.data(), K.out.size() * 8);
+    D->t.log = (const double2*)put(K.log.data(), K.log.size() * 8);
+    D->t.m2m = (const double*)put(K.m2m.data(), K.m2m.size() * 8);
+    D->t.l2l = (const double*)put(K.l2l.data(), K.l2l.size() * 8);
+    D->t.down = (const double2*)put(K.down.data(), K.down.size() * 8);
+    D->t.up = (const double2*)put(K.up.data(), K.up.size() * 8);
+    D->t.zero = (const double2*)put(zero.data(), zero.size() * 8);
+    D->t.dir_vec = (const int*)put(T.dir_vec.data(), T.dir_vec.size() * 4);
+    D->t.class_dirs = (const int*)put(T.class_dirs.data(), T.class_dirs.size() * 4);
+    D->t.m2l32 = (const float2*)put(m2l32.data(), m2l32.size() * 4);
     if (!ok || hipDeviceSynchronize() != hipSuccess) {
         (void)hipFree(blk);
         delete D;
@@ -136,26 +145,31 @@ static int fmm2d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3
     size_t nev = 0;
     int launches = 0, mixed_launches = 0;
     if (far) {
-        for (int l = 2; l < depth; ++l) {
+        M2L2dLevels fp64{};
+        std::vector<M2L2dArgs> fp32;
+        for (int l = depth - 1; l >= 2; --l) {  // the largest first
             M2L2dArgs ma{};
-            ma.N = N;
             ma.level = l;
             ma.num_parents = (int)T.cnt[l - 1];
             ma.child_begin = T.lbegin[l - 1];
             ma.child_keys = T.lkeys[l];
             ma.lut = T.lut[l];
-            ma.keys = T.lkeys[l];
             ma.size = (int)T.cnt[l];
             ma.log_h = std::log(std::ldexp(scale, -l));
             ma.src = outer[l];
-            ma.parent_local = (l > 2) ? inner[l - 1] : nullptr;
             ma.dst = inner[l];
-            ma.f32 = mixed && l >= kMixed2dFirstLevel;
-            mixed_launches += ma.f32 ? 1 : 0;
-            if (timed) LFMM_HIP(hipEventRecord(ctx_event(ctx, nev++), st));
-            LFMM_HIP(launch_m2l2d(ma, DT->t, st));
-            if (timed) LFMM_HIP(hipEventRecord(ctx_event(ctx, nev++), st));
-            ++launches;
+            if (mixed && l >= kMixed2dFirstLevel) fp32.push_back(ma);
+            else fp64.level[fp64.count++] = ma;
+        }
+        if (timed) LFMM_HIP(hipEventRecord(ctx_event(ctx, nev++), st));
+        for (const M2L2dArgs& ma : fp32) LFMM_HIP(launch_m2l2d_f32(N, ma, DT->t, st));
+        LFMM_HIP(launch_m2l2d(N, fp64, DT->t, st));
+        if (timed) LFMM_HIP(hipEventRecord(ctx_event(ctx, nev++), st));
+        mixed_launches = (int)fp32.size();
+        launches = mixed_launches + 1;
+        for (int l = 3; l < depth; ++l) {
+            L2L2dArgs la{N, (int)T.cnt[l - 1], T.lbegin[l - 1], T.lkeys[l], inner[l - 1], inner[l]};
+            LFMM_HIP(launch_l2l2d(la, DT->t, st));
         }
     }
     double t_down = 0.0;
@@ -178,7 +192,17 @@ static int fmm2d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3
     la.nleaf = (int)T.cnt[leaf_level];
     la.level = leaf_level;
     la.geom = T.geom;
-    la.lut = (leaf_level >= 2 && leaf_level <= lut_max_level(2)) ? T.lut[leaf_level] : nullptr;
+    int2* nbr = take<int2>(A, T.cnt[leaf_level] * 9);
+    int32_t* near_total = take<int32_t>(A, T.cnt[leaf_level]);
+    int32_t* near_runs = take<int32_t>(A, T.cnt[leaf_level]);
+    if (!nbr || !near_total || !near_runs) return LFMM_ERR_NOMEM;
+    LFMM_HIP(launch_leaf_ranges(2, la.leaf_key, la.leaf_begin, la.nleaf, leaf_level,
+                                (leaf_level >= 2 && leaf_level <= lut_max_level(2)) ? T.lut[leaf_level] : nullptr, nbr,
+                                near_total, near_runs, st));
+    la.nbr = nbr;
+    la.near_total = near_total;
+    la.near_runs = near_runs;
+    la.wide = scale > 1e150;
     la.local = far ? inner[leaf_level] : nullptr;
     la.N = N;
     la.perm = T.order;

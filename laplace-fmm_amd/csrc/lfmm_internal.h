@@ -76,6 +76,23 @@ struct OpTables2d {
 };
 void build_op_tables_2d(int N, OpTables2d& T);
 
+// Factored form of the 2D operators, every entry a real matrix between two
+// complex diagonals (see pack_2d); complex values interleaved.
+constexpr int m2l2d_blocks(int N) { return N >= 25 ? 3 : N >= 12 ? 2 : 1; }  // row blocks, one per wave
+constexpr int m2l2d_pairs(int N) { return ((N + 1) / 2 + m2l2d_blocks(N) - 1) / m2l2d_blocks(N); }  // row pairs of one
+constexpr int m2l2d_regs(int N) { return (m2l2d_pairs(N) * 2 * N + 15) / 16; }
+struct Pack2d {
+    std::vector<double> m2l;    // [blocks][regs][16]: per row pair and source coefficient, the two rows' entries
+    std::vector<double> src;    // [40][2][32]: re, im of (-1)^j d^-j
+    std::vector<double> out;    // [40][blocks][2][16]: re, im of d^-l, the block's rows
+    std::vector<double> log;    // [40] complex conj(log(-d))
+    std::vector<double> m2m;    // [N][N]: out j, in s
+    std::vector<double> l2l;    // [N][N]: out k, in j
+    std::vector<double> down;   // [N] complex (e/2)^k, e = (1 + i)/2 the class 3 child's offset
+    std::vector<double> up;     // [N] complex e^-k
+};
+void pack_2d(int N, Pack2d& P);
+
 // Dense real form of the M2L operator of direction `dir` (< kNumM2LDirs):
 // K[row * N^2 + col], rows and columns in m2l_real_index order.
 int m2l_real_index(int n, int m, int part);

@@ -35,32 +35,12 @@
 #include "device_common.h"
 #include "m2l_children.h"
 #include "m2lv.h"
+#include "rowbc.h"
 #include "ops3d_kernels.h"
 
 #include <algorithm>
 
 namespace lfmm {
-
-// acc += (entry I of c's 16-lane row) * x
-template <int I>
-__device__ __forceinline__ void fmac_bc(double& acc, double c, double x)
-{
-    asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(I));
-}
-// acc -= (entry I of c's 16-lane row) * x
-template <int I>
-__device__ __forceinline__ void fnmac_bc(double& acc, double c, double x)
-{
-    asm("v_fmac_f64_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(I));
-}
-// entry I of c's 16-lane row in every lane
-template <int I>
-__device__ __forceinline__ double bc(double c)
-{
-    double r;
-    asm("v_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(c), "n"(I));
-    return r;
-}
 
 #define LFMM_BC(I) " row_newbcast:" I " row_mask:0xf bank_mask:0xf"
 // Products with entries I, I + 1, .. of c.  Two rows of a rotation:
@@ -89,15 +69,6 @@ __device__ __forceinline__ void pair_bc(double& a, double& b, double c, double x
     asm("v_fmac_f64_dpp %0, %2, %3" LFMM_BC("%5") "\n\tv_fmac_f64_dpp %1, %2, %4" LFMM_BC("%6")
         : "+&v"(a), "+&v"(b)
         : "v"(c), "v"(x), "v"(y), "n"(I), "n"(J));
-}
-// two output degrees of a translation: re0 += t0 x, im0 += t0 y, re1 += t1 x, im1 += t1 y
-template <int I>
-__device__ __forceinline__ void tr4_bc(double& re0, double& im0, double& re1, double& im1, double c, double x, double y)
-{
-    asm("v_fmac_f64_dpp %0, %4, %5" LFMM_BC("%7") "\n\tv_fmac_f64_dpp %1, %4, %6" LFMM_BC("%7")
-        "\n\tv_fmac_f64_dpp %2, %4, %5" LFMM_BC("%8") "\n\tv_fmac_f64_dpp %3, %4, %6" LFMM_BC("%8")
-        : "+&v"(re0), "+&v"(im0), "+&v"(re1), "+&v"(im1)
-        : "v"(c), "v"(x), "v"(y), "n"(I), "n"(I + 1));
 }
 #undef LFMM_BC
 

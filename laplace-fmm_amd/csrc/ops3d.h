@@ -205,10 +205,6 @@ hipError_t launch_l2p(int N, const LeafArgs& a, hipStream_t st);
 // set.  ws: p2p_ws_elems(n, nleaf) int32; scan_ws: scan_ws_elems(nleaf).
 int64_t p2p_ws_elems(int64_t n, int64_t nleaf);
 hipError_t launch_p2p(const LeafArgs& a, int32_t* ws, uint32_t* scan_ws, hipStream_t st);
-// nbr[leaf][0 .. runs[leaf]) = particle ranges of the 27 neighbour leaves,
-// total[leaf] their particles (tree.hip)
-hipError_t launch_leaf_ranges(const uint64_t* leaf_key, const int32_t* leaf_begin, int nleaf, int level,
-                              const int32_t* lut, int2* nbr, int32_t* total, int32_t* runs, hipStream_t st);
 hipError_t launch_m2l16_pack(int N, const M2L16Args& a, hipStream_t st);
 hipError_t launch_m2l16(int N, const M2L16Args& a, hipStream_t st);
 // dst[i] = (add ? dst[i] : 0) + sum_p partial[p * count + i]   (m2l16.hip)

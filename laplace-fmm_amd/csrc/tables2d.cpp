@@ -103,4 +103,59 @@ void build_op_tables_2d(int N, OpTables2d& T)
     }
 }
 
+// M2L: bt = diag(d^-l) B diag((-1)^j d^-j) at with one real B for every
+// direction (B_lj = C(l+j-1, j-1), column 0: -1/l, row 0: 1), apart from
+// bt_0 += at_0 (log h + conj(log(-d))).  M2M and L2L: child offsets are
+// i^r e, so a child enters M2M as i^(r (j-s)), which depends on (j - s) mod 4
+// alone: the children's four sums with weights i^(r m) go through one real
+// matrix, and the L2L is the transpose.
+void pack_2d(int N, Pack2d& P)
+{
+    OpTables2d T;
+    build_op_tables_2d(N, T);
+    const int ND = (int)T.dir_vec.size() / 2, NB = m2l2d_blocks(N), pairs = m2l2d_pairs(N), regs = m2l2d_regs(N);
+    P.m2l.assign((size_t)NB * regs * 16, 0.0);
+    for (int l = 0; l < N; ++l)
+        for (int j = 0; j < N; ++j) {
+            ld v = 0;
+            if (l == 0) v = j == 0 ? 0 : 1;
+            else v = j == 0 ? -1.0L / (ld)l : binom_l(l + j - 1, j - 1);
+            const int b = l / (2 * pairs), r = l - b * 2 * pairs;
+            P.m2l[(size_t)b * regs * 16 + (size_t)(r / 2) * 2 * N + 2 * j + r % 2] = (double)v;
+        }
+    P.src.assign((size_t)ND * 64, 0.0);
+    P.out.assign((size_t)ND * NB * 32, 0.0);
+    P.log.assign((size_t)ND * 2, 0.0);
+    for (int d = 0; d < ND; ++d) {
+        const cld z((ld)T.dir_vec[2 * d], (ld)T.dir_vec[2 * d + 1]);
+        for (int k = 0; k < N; ++k) {
+            const cld w = 1.0L / cpow_l(z, k);
+            P.src[(size_t)d * 64 + k] = (double)((k & 1) ? -w.real() : w.real());
+            P.src[(size_t)d * 64 + 32 + k] = (double)((k & 1) ? -w.imag() : w.imag());
+            const int b = k / (2 * pairs), r = k - b * 2 * pairs;
+            P.out[((size_t)d * NB + b) * 32 + r] = (double)w.real();
+            P.out[((size_t)d * NB + b) * 32 + 16 + r] = (double)w.imag();
+        }
+        const cld lg = std::conj(std::log(-z));
+        P.log[2 * d] = (double)lg.real();
+        P.log[2 * d + 1] = (double)lg.imag();
+    }
+    const cld e = child_offset(3);
+    P.m2m.assign((size_t)N * N, 0.0);
+    P.l2l.assign((size_t)N * N, 0.0);
+    P.down.assign((size_t)N * 2, 0.0);
+    P.up.assign((size_t)N * 2, 0.0);
+    for (int k = 0; k < N; ++k) {
+        for (int j = 0; j < N; ++j) {
+            P.m2m[(size_t)k * N + j] = (double)(j == 0 ? (k == 0 ? 1.0L : -1.0L / (ld)k) : binom_l(k - 1, j - 1));
+            P.l2l[(size_t)k * N + j] = (double)binom_l(j, k);
+        }
+        const cld a = cpow_l(e / 2.0L, k), b = 1.0L / cpow_l(e, k);
+        P.down[2 * k] = (double)a.real();
+        P.down[2 * k + 1] = (double)a.imag();
+        P.up[2 * k] = (double)b.real();
+        P.up[2 * k + 1] = (double)b.imag();
+    }
+}
+
 }  // namespace lfmm

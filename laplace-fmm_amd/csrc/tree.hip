@@ -546,48 +546,61 @@ __global__ void __launch_bounds__(256) k_count_p2p(const uint64_t* __restrict__ 
 }
 
 // ------------------------------------------------------------------ near-field ranges
-// Half a wave per leaf: lane o < 27 finds the particle range of neighbour o;
-// the ranges are then put in particle order and runs that touch are joined
-// (Morton order: 27 neighbours make 9 to 10 runs on a full tree), so the pair
-// loop changes ranges a third as often and never meets an empty one.
+// A group of lanes per leaf (32 in 3D, 16 in 2D): lane o < 3^D finds the
+// particle range of neighbour o; the ranges are then put in particle order and
+// runs that touch are joined (Morton order: 27 neighbours make 9 to 10 runs on
+// a full tree), so the pair loop changes ranges a third as often and never
+// meets an empty one.
+template <int D>
 __global__ void __launch_bounds__(256) k_leaf_ranges(const uint64_t* __restrict__ leaf_key,
                                                      const int32_t* __restrict__ leaf_begin, int nleaf, int level,
                                                      const int32_t* __restrict__ lut, int2* __restrict__ nbr,
                                                      int32_t* __restrict__ total, int32_t* __restrict__ nruns)
 {
-    __shared__ int2 sorted[8][32];
-    const int half = threadIdx.x >> 5, o = threadIdx.x & 31;
-    const int leaf = blockIdx.x * 8 + half;
+    constexpr int G = D == 3 ? 32 : 16, K = D == 3 ? 27 : 9;
+    __shared__ int2 sorted[256 / G][G];
+    const int group = threadIdx.x / G, o = threadIdx.x % G;
+    const int leaf = blockIdx.x * (256 / G) + group;
     constexpr int kNone = 0x7fffffff;
     int2 r = make_int2(kNone, kNone);
-    if (leaf < nleaf && o < 27) {
+    if (leaf < nleaf && o < K) {
         const uint64_t k = leaf_key[leaf];
-        const int x = (int)compact3(k >> 2) + o / 9 - 1, y = (int)compact3(k >> 1) + (o / 3) % 3 - 1,
-                  z = (int)compact3(k) + o % 3 - 1;
         const int side = 1 << level;
-        if (x >= 0 && y >= 0 && z >= 0 && x < side && y < side && z < side) {
-            const int j = (o == 13) ? leaf : lookup(morton3(x, y, z), lut, leaf_key, nleaf);
+        uint64_t at = 0;
+        bool inside;
+        if constexpr (D == 3) {
+            const int x = (int)compact3(k >> 2) + o / 9 - 1, y = (int)compact3(k >> 1) + (o / 3) % 3 - 1,
+                      z = (int)compact3(k) + o % 3 - 1;
+            inside = x >= 0 && y >= 0 && z >= 0 && x < side && y < side && z < side;
+            if (inside) at = morton3(x, y, z);
+        } else {
+            const int x = (int)compact2(k >> 1) + o / 3 - 1, y = (int)compact2(k) + o % 3 - 1;
+            inside = x >= 0 && y >= 0 && x < side && y < side;
+            if (inside) at = morton2(x, y);
+        }
+        if (inside) {
+            const int j = (o == K / 2) ? leaf : lookup(at, lut, leaf_key, nleaf);
             if (j >= 0) r = make_int2(leaf_begin[j], leaf_begin[j + 1]);
         }
     }
     // rank among the leaf's ranges (begins are distinct, absent ones last)
     int rank = 0;
 #pragma unroll
-    for (int j = 0; j < 32; ++j) {
-        const int bj = __shfl(r.x, j, 32);
+    for (int j = 0; j < G; ++j) {
+        const int bj = __shfl(r.x, j, G);
         rank += (bj < r.x || (bj == r.x && j < o)) ? 1 : 0;
     }
-    sorted[half][rank] = r;
+    sorted[group][rank] = r;
     __syncthreads();
-    r = sorted[half][o];
+    r = sorted[group][o];
     const bool ok = r.x != kNone;
-    const bool head = ok && (o == 0 || sorted[half][o - 1].y != r.x);
-    const bool tail = ok && (o == 31 || sorted[half][o + 1].x != r.y);
-    const uint32_t heads = (uint32_t)(__ballot(head) >> (threadIdx.x & 32));
+    const bool head = ok && (o == 0 || sorted[group][o - 1].y != r.x);
+    const bool tail = ok && (o == G - 1 || sorted[group][o + 1].x != r.y);
+    const uint32_t heads = (uint32_t)(__ballot(head) >> (threadIdx.x & (64 - G))) & (G == 32 ? ~0u : 0xffffu);
     int sum = ok ? r.y - r.x : 0;
-    for (int off = 16; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 32);
-    if (leaf >= nleaf || o >= 27) return;
-    int* out = (int*)(nbr + (int64_t)leaf * 27);
+    for (int off = G / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, G);
+    if (leaf >= nleaf || o >= K) return;
+    int* out = (int*)(nbr + (int64_t)leaf * K);
     if (o == 0) {
         total[leaf] = sum;
         nruns[leaf] = __popc(heads);
@@ -748,12 +761,15 @@ hipError_t count_ops(int dim, const std::vector<uint64_t*>& keys, const std::vec
     return e;
 }
 
-hipError_t launch_leaf_ranges(const uint64_t* leaf_key, const int32_t* leaf_begin, int nleaf, int level,
+hipError_t launch_leaf_ranges(int dim, const uint64_t* leaf_key, const int32_t* leaf_begin, int nleaf, int level,
                               const int32_t* lut, int2* nbr, int32_t* total, int32_t* runs, hipStream_t st)
 {
-    if (nleaf > 0)
-        hipLaunchKernelGGL(k_leaf_ranges, dim3(nblk(nleaf, 8)), dim3(256), 0, st, leaf_key, leaf_begin, nleaf, level, lut, nbr,
-                           total, runs);
+    if (nleaf > 0 && dim == 2)
+        hipLaunchKernelGGL(k_leaf_ranges<2>, dim3(nblk(nleaf, 16)), dim3(256), 0, st, leaf_key, leaf_begin, nleaf, level, lut,
+                           nbr, total, runs);
+    else if (nleaf > 0)
+        hipLaunchKernelGGL(k_leaf_ranges<3>, dim3(nblk(nleaf, 8)), dim3(256), 0, st, leaf_key, leaf_begin, nleaf, level, lut,
+                           nbr, total, runs);
     return hipGetLastError();
 }
 
