@@ -95,7 +95,7 @@ int get_tables(lfmm_ctx* ctx, int N, const DevTables** out)
     D.steps.steps = (const int2*)put(MS.steps.data(), b_ms);
     D.steps.groups = (const int4*)put(MS.groups.data(), b_mg);
     D.steps.zero = (const double2*)put(zero.data(), b_z);
-    for (int c = 0; c < 8; ++c) D.steps.nsteps[c] = MS.nsteps[c];
+    std::copy(MS.nsteps, MS.nsteps + 9, D.steps.nsteps);
     D.m2lv.rot = (const double*)put(V.rot.data(), b_vr);
     D.m2lv.trans = (const double*)put(V.trans.data(), b_vt);
     D.m2lv.ephi = (const double*)put(V.ephi.data(), b_ve);
@@ -108,12 +108,23 @@ int get_tables(lfmm_ctx* ctx, int N, const DevTables** out)
     return LFMM_OK;
 }
 
-// FP64 M2L (with the L2L) of one level: on the vector units while the step
-// state of 64 targets and two tables fit the LDS, on the matrix cores above.
+// FP64 operators of one level: on the vector units while the step state of 64
+// targets and two tables fit the LDS; above that the M2L (with the L2L) on the
+// matrix cores, the M2M and a lone L2L by k_rtr.
+static_assert(LFMM_RTR_MIN_N == kM2lvMaxTerms + 1, "one kernel or the other");
 static int m2l_fp64_tile(int N) { return N <= kM2lvMaxTerms ? kM2lvTile : m64_tile(N); }
+static int rtr_fp64_tile(int N) { return N <= kM2lvMaxTerms ? kM2lvTile : rtr_tile(N); }
 static hipError_t launch_m2l_fp64(int N, const DevTables& D, const M64Level& A, hipStream_t st)
 {
-    return N <= kM2lvMaxTerms ? launch_m2lv(N, D.steps, D.m2lv, A, st) : launch_m2l64(N, D.steps, D.m64, A, st);
+    return N <= kM2lvMaxTerms ? launch_m2lv(N, M2LV_M2L, D.steps, D.m2lv, A, st) : launch_m2l64(N, D.steps, D.m64, A, st);
+}
+static hipError_t launch_m2m_fp64(int N, const DevTables& D, const RtrLevel& L, hipStream_t st)
+{
+    return N <= kM2lvMaxTerms ? launch_m2lv(N, M2LV_M2M, D.steps, D.m2lv, M64Level{L}, st) : launch_rtr(N, 0, D.rt, L, st);
+}
+static hipError_t launch_l2l_fp64(int N, const DevTables& D, const RtrLevel& L, hipStream_t st)
+{
+    return N <= kM2lvMaxTerms ? launch_m2lv(N, M2LV_L2L, D.steps, D.m2lv, M64Level{L}, st) : launch_rtr(N, 2, D.rt, L, st);
 }
 
 // Split-fp16 dense M2L operators of N terms (m2l_dense.cpp), built once per context.
@@ -648,14 +659,14 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
             if (mixed && l >= mfl) L.absmax = xmax + l;
             // small uniform levels: the 8 child classes over 8 parts, summed
             // after (a few tiles alone leave the chip idle)
-            if (!adaptive && !L.absmax && (cnt[l] + rtr_tile(N) - 1) / rtr_tile(N) < 128) {
+            if (!adaptive && !L.absmax && (cnt[l] + rtr_fp64_tile(N) - 1) / rtr_fp64_tile(N) < 128) {
                 L.dsplit = 8;
                 L.size = (int)cnt[l];
                 L.partial = take<double2>(A, 8 * cnt[l] * NX);
                 if (!L.partial) return LFMM_ERR_NOMEM;
             }
             LFMM_HIP(ev_open());
-            LFMM_HIP(launch_rtr(N, 0, DT->rt, L, st));
+            LFMM_HIP(launch_m2m_fp64(N, *DT, L, st));
             if (L.dsplit > 1) LFMM_HIP(launch_sum_parts(L.partial, L.dsplit, cnt[l] * NX, outer[l], false, st));
             LFMM_HIP(ev_close(EV_M2M));
         }
@@ -691,7 +702,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
             L.src = outer[l];
             L.parent_local = (l > first) ? inner[l - 1] : nullptr;
             L.dst = inner[l];
-            L.tiles = (int)((cnt[l - 1] + rtr_tile(N) - 1) / rtr_tile(N));
+            L.tiles = (int)((cnt[l - 1] + rtr_fp64_tile(N) - 1) / rtr_fp64_tile(N));
             const bool bucketed = adaptive && l >= mfl && (per_box || cnt[l - 1] >= kBucketMinParents);
             // FP64 M2L of a large, mostly full level: sources class-major
             double2* vpacked = nullptr;
@@ -731,7 +742,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                     Lb.dsplit = 1;
                     Lb.csorted = 1;
                     for (int c = 0; c <= 8; ++c) Lb.coff[c] = (int)(O.seg[key + c] - b0);
-                    const int tw = mixed ? rtr_tile(t) : m2l_fp64_tile(t);
+                    const int tw = mixed ? rtr_fp64_tile(t) : m2l_fp64_tile(t);
                     Lb.ctile[0] = 0;
                     for (int c = 0; c < 8; ++c)
                         Lb.ctile[c + 1] = Lb.ctile[c] + (Lb.coff[c + 1] - Lb.coff[c] + tw - 1) / tw;
@@ -783,7 +794,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                             m.partial = list_partial;
                         }
                         LFMM_HIP(ev_open());
-                        LFMM_HIP(launch_rtr(t, 2, DB->rt, Lb, st));
+                        LFMM_HIP(launch_l2l_fp64(t, *DB, Lb, st));
                         LFMM_HIP(ev_close(EV_L2L));
                         LFMM_HIP(ev_open());
                         LFMM_HIP(launch_m2l16(t, m, st));
@@ -832,7 +843,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                 }
                 if (lpack.empty()) LFMM_HIP(launch_m2l16_pack(N, m, st));  // else packed in the upward pass
                 LFMM_HIP(ev_open());
-                LFMM_HIP(launch_rtr(N, 2, DT->rt, L, st));
+                LFMM_HIP(launch_l2l_fp64(N, *DT, L, st));
                 LFMM_HIP(ev_close(EV_L2L));
                 LFMM_HIP(ev_open());
                 LFMM_HIP(launch_m2l16(N, m, st));

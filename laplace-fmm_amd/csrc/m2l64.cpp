@@ -72,8 +72,8 @@ void pack_m2l64(const OpTables& T, M64Pack& out)
 // (whose sources stay cache-resident) holds for the groups.
 void pack_m2l_steps(const OpTables& T, M2LSteps& out)
 {
-    out.steps.assign((size_t)8 * kM64Steps * 2, -1);
-    out.groups.assign((size_t)8 * kM64Groups * 4, 0);
+    out.steps.assign((size_t)9 * kM64Steps * 2, -1);
+    out.groups.assign((size_t)9 * kM64Groups * 4, 0);
     for (int c = 0; c < 8; ++c) {
         const int* dirs = &T.class_dirs[c * kDirsPerClass];
         int* st = &out.steps[(size_t)c * kM64Steps * 2];
@@ -111,6 +111,26 @@ void pack_m2l_steps(const OpTables& T, M2LSteps& out)
         }
         out.nsteps[c] = ns;
     }
+    int* st = &out.steps[(size_t)8 * kM64Steps * 2];
+    int* gr = &out.groups[(size_t)8 * kM64Groups * 4];
+    int ns = 0, ng = 0;
+    std::vector<char> used(8, 0);
+    for (int i = 0; i < 8; ++i) {
+        if (used[i]) continue;
+        int* g = gr + 4 * ng++;
+        g[0] = T.dir_theta[kDiagBase + i];
+        g[1] = kTransM2M;
+        g[2] = ns;
+        for (int s = i; s < 8; ++s) {
+            if (used[s] || T.dir_theta[kDiagBase + s] != g[0]) continue;
+            used[s] = 1;
+            st[2 * ns] = kDiagBase + s;
+            st[2 * ns + 1] = 8 * 13 + s;
+            ++ns;
+        }
+        g[3] = ns;
+    }
+    out.nsteps[8] = ns;
 }
 
 }  // namespace lfmm

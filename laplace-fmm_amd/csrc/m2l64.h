@@ -38,16 +38,17 @@ constexpr int kM64MinTerms = 14;                               // smaller expans
 // M2L steps of one target child class, grouped by operator (m2l64.cpp); both
 // FP64 M2L kernels walk them.
 struct M2LSteps {
-    std::vector<int> steps;     // [8][kM64Steps] (direction, 8 * neighbour parent + source class; -1: L2L)
-    std::vector<int> groups;    // [8][kM64Groups] (theta, translation, first step, end)
-    int nsteps[8] = {};
+    // class 8: the M2M of a parent, its children as sources of neighbour parent 13
+    std::vector<int> steps;     // [9][kM64Steps] (direction, 8 * neighbour parent + source class; -1: L2L)
+    std::vector<int> groups;    // [9][kM64Groups] (theta, translation, first step, end)
+    int nsteps[9] = {};
 };
 void pack_m2l_steps(const OpTables& T, M2LSteps& out);
 struct M2LStepTables {
     const int2* steps;
     const int4* groups;
     const double2* zero;        // an expansion of zeros
-    int nsteps[8];
+    int nsteps[9];
 };
 
 // The tables in the operand layout of the FP64 matrix-core M2L (m2l64.cpp).

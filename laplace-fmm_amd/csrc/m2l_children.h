@@ -23,12 +23,13 @@ typedef double m64_v2 __attribute__((ext_vector_type(2)));
 // of target j; targets are the children of the parents pbeg .. pend - 1 of the
 // level or of its list.  An M2L step then finds its source by one LDS read
 // instead of a key interleave, a bounds check and a table lookup per lane.
-template <int TILE, int NT>
+// Entries K0 .. K1 - 1 only (13: the parent itself).
+template <int TILE, int NT, int K0 = 0, int K1 = 27>
 __device__ __forceinline__ void m64_children(const M64Level& A, int pbeg, int pend, int2 (*kids)[TILE])
 {
     const RtrLevel& L = A.L;
     const int pside = 1 << (L.level - 1);
-    for (int e = threadIdx.x; e < 27 * TILE; e += NT) {
+    for (int e = K0 * TILE + threadIdx.x; e < K1 * TILE; e += NT) {
         const int k = e / TILE, j = e - k * TILE;
         int2 v = make_int2(0, 0);
         if (pbeg + j < pend) {

@@ -4,14 +4,14 @@
 
 namespace lfmm {
 
-template <int N> hipError_t do_m2lv(const M2LStepTables& S, const M2lvTables& V, const M64Level& A, hipStream_t st);
+template <int N> hipError_t do_m2lv(int op, const M2LStepTables& S, const M2lvTables& V, const M64Level& A, hipStream_t st);
 
 #define LFMM_M2LV_TERMS(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13)
 
-hipError_t launch_m2lv(int N, const M2LStepTables& S, const M2lvTables& V, const M64Level& A, hipStream_t st)
+hipError_t launch_m2lv(int N, int op, const M2LStepTables& S, const M2lvTables& V, const M64Level& A, hipStream_t st)
 {
     switch (N) {
-#define X(n) case n: return do_m2lv<n>(S, V, A, st);
+#define X(n) case n: return do_m2lv<n>(op, S, V, A, st);
         LFMM_M2LV_TERMS(X)
 #undef X
     default: return hipErrorInvalidValue;

@@ -113,6 +113,8 @@ struct M2lvTables {
 // absent children and from slot num_parents on.
 inline int m2lv_slots(int64_t parents) { return (int)((parents + 8) / 8 * 8); }
 hipError_t launch_m2lv_pack(const RtrLevel& L, int nx, double2* packed, hipStream_t st);
-hipError_t launch_m2lv(int N, const M2LStepTables& S, const M2lvTables& V, const M64Level& A, hipStream_t st);
+// op: M2LV_M2L, M2LV_M2M (A.L as for launch_rtr) or M2LV_L2L
+enum { M2LV_M2L = 0, M2LV_M2M = 1, M2LV_L2L = 2 };
+hipError_t launch_m2lv(int N, int op, const M2LStepTables& S, const M2lvTables& V, const M64Level& A, hipStream_t st);
 
 }  // namespace lfmm

@@ -1,7 +1,7 @@
-// m2lv_kernels.h -- FP64 M2L (fused with L2L) of up to 13 terms on the vector
-// units: the rotate / axial-translate / rotate-back operator (reference M2L
-// :152-190, L2L :192-226 and Downward :328-349 of src/cpu/multipole3d.cpp).
-// Compiled once per expansion size.
+// m2lv_kernels.h -- FP64 M2L (fused with L2L), M2M and L2L of up to 13 terms on
+// the vector units: the rotate / axial-translate / rotate-back operator
+// (reference M2M :115-150, M2L :152-190, L2L :192-226 and Downward :328-349 of
+// src/cpu/multipole3d.cpp).  Compiled once per expansion size.
 //
 // A workgroup owns 64 targets, one per lane, and walks their interaction
 // directions.  The state of a direction lives in LDS as [coefficient][lane]
@@ -136,7 +136,11 @@ __device__ __forceinline__ void m2lv_rows(M2lvStream<REGS>& S, const double2 (&v
     });
 }
 
-template <int N, int NW, int W, bool PACKED>
+// OP: M2L with the L2L, or one of the other two operators of this form alone:
+// M2M (targets: parents, steps: their 8 children) and L2L (one step).  With
+// scalar coefficients (k_rtr) a step took 12 us however few the boxes; here,
+// 13 terms, 4M clustered particles: M2M 2.40 -> 1.12 ms, L2L 0.79 -> 0.51.
+template <int N, int NW, int W, bool PACKED, int OP>
 __device__ __forceinline__ void m2lv_wave(const M2LStepTables& T, const M2lvTables& V, const M64Level& A, double2* state,
                                           double (*tab)[M2lvBuf<N, NW>::size], m2lv_near_t<PACKED> (*near)[kM2lvTile],
                                           int c, int part, int pbeg, int pend)
@@ -157,13 +161,17 @@ __device__ __forceinline__ void m2lv_wave(const M2LStepTables& T, const M2lvTabl
         else return (v.y >> (ks & 7)) & 1 ? v.x + __popc(v.y & ((1 << (ks & 7)) - 1)) : -1;
     };
     int tgt = -1;
-    if (P >= 0)
+    if constexpr (OP == M2LV_M2M) {
+        // a parent without children (a leaf of the adaptive tree) keeps its P2M
+        if (P >= 0 && L.child_begin[P + 1] > L.child_begin[P]) tgt = P;
+    } else if (P >= 0) {
         for (int i = L.child_begin[P]; i < L.child_begin[P + 1]; ++i)
             if ((int)(L.child_keys[i] & 7u) == c) tgt = i;
-    const int g_first = L.parent_local ? 0 : 1;
+    }
+    const int g_first = OP == M2LV_M2L && !L.parent_local ? 1 : 0;
     const auto groups = m64_scalar((const m64_i4*)T.groups) + c * kM64Groups;  // (theta, translation, first step, end)
     const auto steps = m64_scalar((const m64_i2*)T.steps) + c * kM64Steps;     // (direction, 8 * neighbour parent + source class)
-    const int s_first = groups[g_first].z, ns = T.nsteps[c] - s_first;
+    const int s_first = groups[g_first].z, ns = OP == M2LV_L2L ? 1 : T.nsteps[c] - s_first;
     const int d_beg = s_first + part * ns / L.dsplit, d_end = s_first + (part + 1) * ns / L.dsplit;
     int gi = g_first;
     while (groups[gi].w <= d_beg) ++gi;
@@ -340,6 +348,7 @@ __device__ __forceinline__ void m2lv_wave(const M2LStepTables& T, const M2lvTabl
             buf ^= 1;
         }
     }
+    double mx = 0.0;
     if (tgt >= 0) {
         double2* out = L.dsplit > 1 ? L.partial + ((int64_t)part * L.size + tgt) * NX : L.dst + (int64_t)tgt * SX;
         if constexpr (W == 0)  // coefficients beyond this launch's order are zero
@@ -351,12 +360,15 @@ __device__ __forceinline__ void m2lv_wave(const M2LStepTables& T, const M2lvTabl
                     constexpr int m = decltype(M)::value;
                     const double2 v = acc[tri(n) + m];
                     out[tri(n) + m] = (m & 1) ? make_double2(-v.x, -v.y) : v;
+                    if constexpr (OP == M2LV_M2M) mx = fmax(mx, fmax(fabs(v.x), fabs(v.y)));
                 });
         });
     }
+    if constexpr (OP == M2LV_M2M)
+        if (L.absmax) wave_absmax(mx, L.absmax);
 }
 
-template <int N, int NW, bool PACKED>
+template <int N, int NW, bool PACKED, int OP = M2LV_M2L>
 __global__ void __launch_bounds__(64 * NW, 2) k_m2lv(M2LStepTables T, M2lvTables V, M64Level A)
 {
     using B = M2lvBuf<N, NW>;
@@ -366,7 +378,11 @@ __global__ void __launch_bounds__(64 * NW, 2) k_m2lv(M2LStepTables T, M2lvTables
     const RtrLevel& L = A.L;
     const int blk = xcd_local_block(blockIdx.x, gridDim.x);
     int tile, c, part = 0, pbeg = 0, pend = L.num_parents;
-    if (L.csorted) {
+    if constexpr (OP == M2LV_M2M) {
+        tile = blk / L.dsplit;
+        part = blk - tile * L.dsplit;
+        c = 8;  // of the step tables
+    } else if (L.csorted) {
         c = blk & 7;
         tile = blk >> 3;
         if (tile >= L.ctile[c + 1] - L.ctile[c]) return;  // the whole block
@@ -381,21 +397,27 @@ __global__ void __launch_bounds__(64 * NW, 2) k_m2lv(M2LStepTables T, M2lvTables
     }
     pbeg += tile * kM2lvTile;
     if constexpr (PACKED) m64_parents<kM2lvTile, 64 * NW>(A, pbeg, pend, near);
-    else m64_children<kM2lvTile, 64 * NW>(A, pbeg, pend, near);
+    else if constexpr (OP == M2LV_M2L) m64_children<kM2lvTile, 64 * NW>(A, pbeg, pend, near);
+    else if constexpr (OP == M2LV_M2M) m64_children<kM2lvTile, 64 * NW, 13, 14>(A, pbeg, pend, near);
     __syncthreads();
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     sfor<0, NW>([&](auto WW) {
         constexpr int W = decltype(WW)::value;
-        if (w == W) m2lv_wave<N, NW, W, PACKED>(T, V, A, state, tab, near, c, part, pbeg, pend);
+        if (w == W) m2lv_wave<N, NW, W, PACKED, OP>(T, V, A, state, tab, near, c, part, pbeg, pend);
     });
 }
 
 template <int N>
-hipError_t do_m2lv(const M2LStepTables& T, const M2lvTables& V, const M64Level& A, hipStream_t st)
+hipError_t do_m2lv(int op, const M2LStepTables& T, const M2lvTables& V, const M64Level& A, hipStream_t st)
 {
+    constexpr int NW = m2lv_nw(N);
     const RtrLevel& L = A.L;
+    const int tiles = (L.num_parents + kM2lvTile - 1) / kM2lvTile;
     int blocks = 0;
-    if (L.csorted) {
+    if (op == M2LV_M2M) {
+        if (L.plist || L.csorted || L.dsplit < 1 || L.dsplit > 8) return hipErrorInvalidValue;
+        blocks = tiles * L.dsplit;
+    } else if (L.csorted) {
         if (L.dsplit != 1 || !L.plist || L.coff[8] != L.num_parents) return hipErrorInvalidValue;
         int mt = 0;
         for (int c = 0; c < 8; ++c) {
@@ -405,13 +427,15 @@ hipError_t do_m2lv(const M2LStepTables& T, const M2lvTables& V, const M64Level& 
         }
         blocks = 8 * mt;
     } else {
-        if (L.tiles != (L.num_parents + kM2lvTile - 1) / kM2lvTile) return hipErrorInvalidValue;
+        if (L.tiles != tiles || (op == M2LV_L2L && L.dsplit != 1)) return hipErrorInvalidValue;
         blocks = L.tiles * 8 * L.dsplit;
     }
-    if (blocks > 0) {
-        if (A.packed) hipLaunchKernelGGL((k_m2lv<N, m2lv_nw(N), true>), dim3(blocks), dim3(64 * m2lv_nw(N)), 0, st, T, V, A);
-        else hipLaunchKernelGGL((k_m2lv<N, m2lv_nw(N), false>), dim3(blocks), dim3(64 * m2lv_nw(N)), 0, st, T, V, A);
-    }
+    if (blocks <= 0) return hipSuccess;
+    const dim3 grid(blocks), block(64 * NW);
+    if (op == M2LV_M2M) hipLaunchKernelGGL((k_m2lv<N, NW, false, M2LV_M2M>), grid, block, 0, st, T, V, A);
+    else if (op == M2LV_L2L) hipLaunchKernelGGL((k_m2lv<N, NW, false, M2LV_L2L>), grid, block, 0, st, T, V, A);
+    else if (A.packed) hipLaunchKernelGGL((k_m2lv<N, NW, true>), grid, block, 0, st, T, V, A);
+    else hipLaunchKernelGGL((k_m2lv<N, NW, false>), grid, block, 0, st, T, V, A);
     return hipGetLastError();
 }
 

@@ -35,9 +35,10 @@ hipError_t launch_p2l(int N, const P2MArgs& a, hipStream_t st)
 
 hipError_t launch_rtr(int N, int kind, const RtrTables& T, const RtrLevel& L, hipStream_t st)
 {
+    static_assert(LFMM_RTR_MIN_N == 14, "the sizes below");
     switch (N) {
 #define X(n) case n: return do_rtr<n>(kind, T, L, st);
-        LFMM_FOR_TERMS(X)
+        X(14) X(15) X(16) X(17) X(18)
 #undef X
     default: return hipErrorInvalidValue;
     }

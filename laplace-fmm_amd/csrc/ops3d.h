@@ -198,6 +198,8 @@ constexpr int m16_targets(int N)
 hipError_t launch_p2m(int N, const P2MArgs& a, hipStream_t st);
 // P2L of one level's X lists (adaptive octree; see P2MArgs)
 hipError_t launch_p2l(int N, const P2MArgs& a, hipStream_t st);
+// M2M (kind 0) and L2L (2) from LFMM_RTR_MIN_N terms on; below, launch_m2lv
+#define LFMM_RTR_MIN_N 14
 hipError_t launch_rtr(int N, int kind, const RtrTables& T, const RtrLevel& L, hipStream_t st);
 // L2P alone into a.far (k_l2p), for the pair kernels below
 hipError_t launch_l2p(int N, const LeafArgs& a, hipStream_t st);

@@ -2,8 +2,9 @@
 // Compiled once per expansion size by ops3d_inst.hip (-DLFMM_N=<terms>).
 //
 //   k_p2m   P2M, wave per leaf           (reference Multipole, src/cpu/multipole3d.cpp:20-49)
-//   k_rtr   M2M and L2L                  (reference M2M :115-150, L2L :192-226); the M2L is in
-//           m2lv_kernels.h, m2l64_kernels.h (FP64) and m2l16_kernels.h (split FP16)
+//   k_rtr   M2M and L2L from 14 terms on (reference M2M :115-150, L2L :192-226); below, both
+//           are in m2lv_kernels.h; the M2L is in m2lv_kernels.h, m2l64_kernels.h (FP64) and
+//           m2l16_kernels.h (split FP16)
 //   k_l2p   L2P, lane per target particle, far field in sorted order
 //           (reference ComputeLeaves<double> :1156-1210); the pair sums and the
 //           scatter to input order are in p2p.hip
