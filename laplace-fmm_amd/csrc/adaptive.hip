@@ -82,6 +82,7 @@ __device__ inline int uni_level(const UniLevels& U, int j)
 struct AdInfo {
     int32_t loff[kAdMaxLevels + 1];  // first box of each level
     uint32_t max_leaf;
+    int32_t ioff[kAdMaxLevels + 1];  // boxes with children before each level
     uint32_t nleaf, fine_pairs, x_pairs, u_total, n_total;
     uint32_t xseg[kAdMaxLevels + 1];
 };
@@ -391,6 +392,37 @@ __global__ void __launch_bounds__(256) k_ad_near_fill(const int32_t* __restrict_
     }
 }
 
+// boxes with children: numbered within their level (slot, -1: none) and
+// listed (list: index at the level, levels one after another)
+struct AdInner {
+    const int32_t* box2leaf;
+    int64_t n;
+    __device__ uint32_t operator()(int64_t g) const { return g < n && box2leaf[g] < 0 ? 1u : 0u; }
+};
+
+struct AdInnerOut {
+    AdLevels A;
+    const int32_t* box2leaf;
+    int64_t n;
+    uint32_t* before_all;
+    int32_t* list;
+    AdInfo* host;
+    __device__ void operator()(int64_t g, uint32_t before) const
+    {
+        before_all[g] = before;
+        for (int l = 0; l <= A.depth; ++l)
+            if (g == A.off[l]) host->ioff[l] = (int32_t)before;
+        if (g < n && box2leaf[g] < 0) list[before] = (int32_t)g - A.off[ad_level(A, (int)g)];
+    }
+};
+
+__global__ void __launch_bounds__(256) k_ad_slots(AdLevels A, const int32_t* __restrict__ box2leaf, int n,
+                                                  const uint32_t* __restrict__ before, int32_t* __restrict__ slot)
+{
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g < n) slot[g] = box2leaf[g] < 0 ? (int32_t)(before[g] - before[A.off[ad_level(A, g)]]) : -1;
+}
+
 // ---- inputs and outputs of the scans: counts of `live` entries (then zeros)
 // into offsets; the total goes to the host
 struct AdCount {
@@ -599,6 +631,13 @@ int build_adaptive(lfmm_ctx* ctx, int leaf_max, Tree& T, int min_leaf_level)
                        nleaf, nbr27, nu1, nco, most);
     rc = scan_to(A, AdCount{nco, nleaf, 0}, AdOffsets{coff, total, &info->fine_pairs, most, &info->max_leaf}, total, st);
     if (rc != LFMM_OK) return rc;
+    uint32_t* inner_before = take<uint32_t>(A, total + 1);
+    T.inner_list = take<int32_t>(A, total);
+    T.inner_slot = take<int32_t>(A, total);
+    if (!inner_before || !T.inner_list || !T.inner_slot) return LFMM_ERR_NOMEM;
+    rc = scan_to(A, AdInner{T.box2leaf, total}, AdInnerOut{V, T.box2leaf, total, inner_before, T.inner_list, info}, total, st);
+    if (rc != LFMM_OK) return rc;
+    hipLaunchKernelGGL(k_ad_slots, dim3(nblk(total, 256)), dim3(256), 0, st, V, T.box2leaf, total, inner_before, T.inner_slot);
     const int g2 = depth > 2 ? T.loff[2] : total;
     const int nb = total - g2;
     int32_t* x27 = nullptr;
@@ -619,6 +658,7 @@ int build_adaptive(lfmm_ctx* ctx, int leaf_max, Tree& T, int min_leaf_level)
     LFMM_HIP(hipStreamSynchronize(st));
     const int64_t nl = T.nleaf = info->nleaf;
     T.max_leaf = info->max_leaf;
+    T.ioff.assign(info->ioff, info->ioff + depth + 1);
     const int64_t npairs = info->fine_pairs;
     T.x_pairs = info->x_pairs;
     T.xseg.assign(depth + 1, 0);

@@ -657,6 +657,18 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
             L.src = outer[l + 1];
             L.dst = outer[l];
             if (mixed && l >= mfl) L.absmax = xmax + l;
+            // an adaptive level: the boxes with children alone
+            const bool listed = adaptive && N <= kM2lvMaxTerms;
+            if (listed) {
+                L.plist = T.inner_list + T.ioff[l];
+                L.num_parents = T.ioff[l + 1] - T.ioff[l];
+                if ((L.num_parents + kM2lvTile - 1) / kM2lvTile < 128) {
+                    L.dsplit = 8;
+                    L.size = L.num_parents;
+                    L.partial = take<double2>(A, (int64_t)8 * L.num_parents * NX);
+                    if (!L.partial) return LFMM_ERR_NOMEM;
+                }
+            }
             // small uniform levels: the 8 child classes over 8 parts, summed
             // after (a few tiles alone leave the chip idle)
             if (!adaptive && !L.absmax && (cnt[l] + rtr_fp64_tile(N) - 1) / rtr_fp64_tile(N) < 128) {
@@ -667,7 +679,10 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
             }
             LFMM_HIP(ev_open());
             LFMM_HIP(launch_m2m_fp64(N, *DT, L, st));
-            if (L.dsplit > 1) LFMM_HIP(launch_sum_parts(L.partial, L.dsplit, cnt[l] * NX, outer[l], false, st));
+            if (L.dsplit > 1 && listed)
+                LFMM_HIP(launch_sum_parent_parts(L.partial, L.dsplit, L.num_parents, NX, L.plist, outer[l], L.absmax, st));
+            else if (L.dsplit > 1)
+                LFMM_HIP(launch_sum_parts(L.partial, L.dsplit, cnt[l] * NX, outer[l], false, st));
             LFMM_HIP(ev_close(EV_M2M));
         }
     }
@@ -687,6 +702,14 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                 big = std::max<int64_t>(big, m2lv_slots(cnt[l - 1]));
         if (big > 0 && !(vpack = take<double2>(A, 8 * NX * big))) return LFMM_ERR_NOMEM;
     }
+    // sources of an adaptive level packed by the parents with children alone
+    // (4M clustered particles: a quarter of all; packing 0.80 -> 0.34 ms, whole
+    // solve 17.8 -> 16.7 with the M2M on the same lists)
+    auto slots_of = [&](M2L16Args& m, int l) {
+        m.slots = T.ioff[l] - T.ioff[l - 1];
+        m.slot = T.inner_slot + T.loff[l - 1];
+        m.slot_parents = T.inner_list + T.ioff[l - 1];
+    };
     double2* list_partial = nullptr;  // direction parts of the matrix-core M2L buckets
     int64_t list_partial_elems = 0;
     if (far) {
@@ -726,6 +749,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                     mp.xp = xp;
                     mp.stride = NX;
                     mp.size = L.size;
+                    slots_of(mp, l);
                     LFMM_HIP(launch_m2l16_pack(tpack, mp, st));
                 }
                 // one launch per order among the level's boxes ((parent, class) lists)
@@ -778,6 +802,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                             m.ctile[c + 1] = m.ctile[c] + (m.coff[c + 1] - m.coff[c] + m16_targets(t) - 1) / m16_targets(t);
                         m.tiles = m.ctile[8];
                         m.xpieces = 4 * ((tpack * tpack + 15) / 16);
+                        if (m16_rowfull(tpack)) slots_of(m, l);
                         // a workgroup runs all 189 directions of its targets:
                         // small buckets split the directions into parts so
                         // that about 512 workgroups share the work

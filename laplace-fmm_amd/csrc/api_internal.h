@@ -166,6 +166,11 @@ struct Tree {
     uint64_t* keys_all = nullptr;     // [total] (lkeys[l] = keys_all + loff[l])
     int2* range_all = nullptr;        // [total] particle range of each box
     int32_t* box2leaf = nullptr;      // [total] leaf index or -1
+    // boxes with children: level l's are inner_list[ioff[l] .. ioff[l + 1]) (indices at
+    // the level); inner_slot[gid]: the place in that list, -1 for a leaf
+    std::vector<int> ioff;
+    int32_t* inner_list = nullptr;
+    int32_t* inner_slot = nullptr;
     int64_t nleaf = 0;                // global leaf list, in particle order:
     int32_t* leaf_begin = nullptr;    //   [nleaf + 1] first particle
     int32_t* leaf_gid = nullptr;      //   [nleaf] box

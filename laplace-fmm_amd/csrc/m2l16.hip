@@ -1,4 +1,5 @@
 // m2l16.hip -- level-wide helpers of the matrix-core M2L.
+#include "device_common.h"
 #include "lfmm_internal.h"
 #include "ops3d.h"
 
@@ -37,6 +38,35 @@ hipError_t launch_sum_parts(const double2* partial, int parts, int64_t count, do
 {
     const int64_t blocks = std::min<int64_t>((count + 255) / 256, 8192);
     if (blocks > 0) hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)blocks), dim3(256), 0, st, partial, parts, count, dst, add ? 1 : 0);
+    return hipGetLastError();
+}
+
+__global__ void __launch_bounds__(256) k_sum_parent_parts(const double2* __restrict__ partial, int parts, int count, int nx,
+                                                          const int32_t* __restrict__ list, double2* __restrict__ dst,
+                                                          uint32_t* __restrict__ absmax)
+{
+    const int64_t total = (int64_t)count * nx, i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    double mx = 0.0;
+    if (i < total) {
+        double2 v = make_double2(0.0, 0.0);
+        for (int p = 0; p < parts; ++p) {
+            const double2 x = partial[p * total + i];
+            v.x += x.x;
+            v.y += x.y;
+        }
+        dst[(int64_t)list[i / nx] * nx + i % nx] = v;
+        mx = fmax(fabs(v.x), fabs(v.y));
+    }
+    if (absmax) wave_absmax(mx, absmax);
+}
+
+hipError_t launch_sum_parent_parts(const double2* partial, int parts, int count, int nx, const int32_t* list, double2* dst,
+                                   uint32_t* absmax, hipStream_t st)
+{
+    const int64_t blocks = ((int64_t)count * nx + 255) / 256;
+    if (blocks > 0)
+        hipLaunchKernelGGL(k_sum_parent_parts, dim3((unsigned)blocks), dim3(256), 0, st, partial, parts, count, nx, list, dst,
+                           absmax);
     return hipGetLastError();
 }
 

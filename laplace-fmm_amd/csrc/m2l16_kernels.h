@@ -101,7 +101,7 @@ __global__ void __launch_bounds__(256) k_m2l16_pack(const double2* __restrict__ 
 // Packs a level's normalised multipoles class-major for k_m2l16r:
 // piece (kc, hi/lo, half) of the class-c child of parent P lands at
 // xp[(c * PIECES + 4 kc + 2 hl + half) * (num_parents + 1) + P], zeros where
-// the child is absent and in slot num_parents.  For one direction, the
+// the child is absent and in slot num_parents (with a list, P is its entry).  For one direction, the
 // sources of a tile's targets are one class and a shifted block of parents,
 // so a source fragment reads runs of consecutive 16-byte entries.
 // A thread packs one (parent, kc, half): the 2 KC threads of a parent are
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(256) k_m2l16_pack_cls(const double2* __restric
                                                         const int32_t* __restrict__ child_begin,
                                                         const uint64_t* __restrict__ child_keys,
                                                         const uint32_t* __restrict__ xmax, uint4* __restrict__ xp,
-                                                        int64_t stride)
+                                                        int64_t stride, const int32_t* __restrict__ list)
 {
     using S = M16<N>;
     const int64_t np1 = (int64_t)num_parents + 1;
@@ -128,8 +128,9 @@ __global__ void __launch_bounds__(256) k_m2l16_pack_cls(const double2* __restric
     // in flight together
     int cb = 0, ce = 0;
     if (P < num_parents) {
-        cb = child_begin[P];
-        ce = child_begin[P + 1];
+        const int64_t Q = list ? list[P] : P;
+        cb = child_begin[Q];
+        ce = child_begin[Q + 1];
     }
     int kcls[8];
 #pragma unroll
@@ -515,6 +516,7 @@ __global__ void __launch_bounds__(256, CTW == 1 ? 2 : 1) k_m2l16r(M2L16Args a, c
                 const int pside = side >> 1;
                 if (px >= 0 && py >= 0 && pz >= 0 && px < pside && py < pside && pz < pside)
                     v = find_box(morton3(px, py, pz), a.plut, a.pkeys, a.num_parents);
+                if (a.slot && v >= 0) v = a.slot[v];
             }
             near[k][e % TC] = v;
         }
@@ -532,7 +534,7 @@ __global__ void __launch_bounds__(256, CTW == 1 ? 2 : 1) k_m2l16r(M2L16Args a, c
     // source of column tile ct in direction dir, as the offset of its class
     // plane entry: class * PIECES * (num_parents + 1) + parent slot (the zero
     // slot num_parents of class 0 when the source or its parent is absent)
-    const int64_t np1 = M2M ? a.src_np1 : (int64_t)a.num_parents + 1;
+    const int64_t np1 = M2M ? a.src_np1 : (int64_t)(a.slot ? a.slots : a.num_parents) + 1;
     const int64_t zslot = np1 - 1;  // the zero entry
     const int64_t xpc = a.xpieces > 0 ? a.xpieces : PIECES;  // pieces per packed box
     auto box_of = [&](int step, int ct) -> int64_t {
@@ -825,10 +827,11 @@ template <int N>
 hipError_t do_m2l16_pack(const M2L16Args& a, hipStream_t st)
 {
     if constexpr (m16_rowfull(N)) {
-        const int64_t packs = ((int64_t)a.num_parents + 1) * M16<N>::KC * 2;
+        const int parents = a.slot ? a.slots : a.num_parents;
+        const int64_t packs = ((int64_t)parents + 1) * M16<N>::KC * 2;
         hipLaunchKernelGGL((k_m2l16_pack_cls<N>), dim3((unsigned)((packs + 255) / 256)), dim3(256), 0, st, a.outer,
-                           a.num_parents, a.child_begin, a.child_keys, a.xmax, a.xp,
-                           (int64_t)(a.stride > 0 ? a.stride : tri(N)));
+                           parents, a.child_begin, a.child_keys, a.xmax, a.xp,
+                           (int64_t)(a.stride > 0 ? a.stride : tri(N)), a.slot ? a.slot_parents : nullptr);
     } else {
         const int64_t packs = (int64_t)(a.size + 1) * M16<N>::KC * 2;
         hipLaunchKernelGGL((k_m2l16_pack<N>), dim3((unsigned)((packs + 255) / 256)), dim3(256), 0, st, a.outer,

@@ -350,7 +350,8 @@ __device__ __forceinline__ void m2lv_wave(const M2LStepTables& T, const M2lvTabl
     }
     double mx = 0.0;
     if (tgt >= 0) {
-        double2* out = L.dsplit > 1 ? L.partial + ((int64_t)part * L.size + tgt) * NX : L.dst + (int64_t)tgt * SX;
+        const int at = OP == M2LV_M2M && L.plist ? pbeg + lane : tgt;  // of a part: list entry or box
+        double2* out = L.dsplit > 1 ? L.partial + ((int64_t)part * L.size + at) * NX : L.dst + (int64_t)tgt * SX;
         if constexpr (W == 0)  // coefficients beyond this launch's order are zero
             for (int64_t i = NX; i < SX; ++i) out[i] = make_double2(0.0, 0.0);
         sfor<0, N>([&](auto NN) {
@@ -365,7 +366,7 @@ __device__ __forceinline__ void m2lv_wave(const M2LStepTables& T, const M2lvTabl
         });
     }
     if constexpr (OP == M2LV_M2M)
-        if (L.absmax) wave_absmax(mx, L.absmax);
+        if (L.absmax && L.dsplit == 1) wave_absmax(mx, L.absmax);  // of parts: with their sum
 }
 
 template <int N, int NW, bool PACKED, int OP = M2LV_M2L>
@@ -415,7 +416,7 @@ hipError_t do_m2lv(int op, const M2LStepTables& T, const M2lvTables& V, const M6
     const int tiles = (L.num_parents + kM2lvTile - 1) / kM2lvTile;
     int blocks = 0;
     if (op == M2LV_M2M) {
-        if (L.plist || L.csorted || L.dsplit < 1 || L.dsplit > 8) return hipErrorInvalidValue;
+        if (L.csorted || L.dsplit < 1 || L.dsplit > 8) return hipErrorInvalidValue;
         blocks = tiles * L.dsplit;
     } else if (L.csorted) {
         if (L.dsplit != 1 || !L.plist || L.coff[8] != L.num_parents) return hipErrorInvalidValue;

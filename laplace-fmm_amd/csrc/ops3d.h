@@ -167,6 +167,12 @@ struct M2L16Args {
     // columns beyond them are zero, so one packing serves every order up to
     // the packed one.
     int xpieces = 0;
+    // k_m2l16r on an adaptive tree: sources are packed by the parents with
+    // children alone, slots of them (0: every parent): slot_parents lists
+    // them, slot maps a parent to its place (-1: none)
+    int slots = 0;
+    const int32_t* slot = nullptr;
+    const int32_t* slot_parents = nullptr;
     // M2M mode (k_m2l16r only): the targets are the boxes of `level` (the
     // class-c children of the num_parents boxes above them, as for M2L), the
     // 8 "directions" are the M2M operators from their children of class
@@ -202,6 +208,11 @@ hipError_t launch_p2l(int N, const P2MArgs& a, hipStream_t st);
 #define LFMM_RTR_MIN_N 14
 hipError_t launch_rtr(int N, int kind, const RtrTables& T, const RtrLevel& L, hipStream_t st);
 // L2P alone into a.far (k_l2p), for the pair kernels below
+// M2M of the listed parents, split over parts: part p of list entry i is at
+// partial + (p * count + i) * nx, their sum goes to dst + list[i] * nx (and its
+// largest |coefficient| to absmax)
+hipError_t launch_sum_parent_parts(const double2* partial, int parts, int count, int nx, const int32_t* list, double2* dst,
+                                   uint32_t* absmax, hipStream_t st);
 hipError_t launch_l2p(int N, const LeafArgs& a, hipStream_t st);
 // Near field with several targets per lane (p2p.hip), starting from a.far when
 // set.  ws: p2p_ws_elems(n, nleaf) int32; scan_ws: scan_ws_elems(nleaf).
