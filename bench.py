@@ -240,7 +240,7 @@ def main():
     else:
         launches = reports[0]["m2l_launches"]
         ach = counts["m2l_ops"] * alg / (m2l_ms * 1e-3) / 1e12
-        roofline = {"kernel": "k_rtr<N,M2L> (M2L+L2L, one launch per level)", "bound": "mfma",
+        roofline = {"kernel": "k_m2lv<N> / k_m2l64<N> (M2L+L2L, one launch per level)", "bound": "mfma",
                     "achieved": round(ach, 3), "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                     "frac": round(ach / FP64_PEAK_TFLOPS, 4), "traffic": None,
                     "flops_counted": "algorithmic rotation-based M2L flops", "m2l_ops": counts["m2l_ops"],
@@ -272,9 +272,9 @@ def main():
                        kernel="k_p2p_multi<2> with its lane setup",
                        bytes_counted="32 B per near-list source per leaf + 32 B target + 32 B far field + 32 B out"),
            "m2m": dict(rate(counts["m2m_bytes"], mean_of(reports, "t_m2m_ms")),
-                       kernel="k_m2l16r<N,CTW,true> (M2M into levels >= 4 on the matrix cores) + k_rtr<N,M2M> (FP64, levels 2-3)",
+                       kernel="k_m2l16r<N,CTW,true> (M2M into levels >= 4 on the matrix cores) + k_m2lv<N> (FP64, levels 2-3)",
                        bytes_counted="every multipole of levels >= 3 read once, levels >= 2 written once"),
-           "l2l": dict(rate(counts["l2l_bytes"], mean_of(reports, "t_l2l_ms")), kernel="k_rtr<N,L2L>",
+           "l2l": dict(rate(counts["l2l_bytes"], mean_of(reports, "t_l2l_ms")), kernel="k_m2lv<N> (L2L alone)",
                        bytes_counted="parent locals read once, child locals written once (levels >= 4)")}
     p2p_pairs = counts["p2p_pairs"]
     leaf = {"kernel": "k_l2p<N> + k_p2p (L2P, then P2P)", "ms_per_step": round(leaf_ms, 4), "p2p_pairs": p2p_pairs,
