@@ -356,7 +356,8 @@ __global__ void __launch_bounds__(256) k_ad_near_fill(const int32_t* __restrict_
                                                       const int32_t* __restrict__ w_gid, const int2* __restrict__ range,
                                                       int direct_max, const uint32_t* __restrict__ n_off,
                                                       int2* __restrict__ n_rng, int32_t* __restrict__ n_sources,
-                                                      int32_t* __restrict__ n_runs)
+                                                      int32_t* __restrict__ n_runs, int32_t* __restrict__ m2p_gid,
+                                                      int32_t* __restrict__ m2p_count)
 {
     const int i = blockIdx.x * kHalves + threadIdx.x / kHalf;
     const uint32_t o = threadIdx.x & 31;
@@ -374,11 +375,15 @@ __global__ void __launch_bounds__(256) k_ad_near_fill(const int32_t* __restrict_
     };
     copy(u_rng + u_off[i], u_off[i + 1] - u_off[i]);
     if (x_off && g >= g2) copy(x_rng + x_off[g - g2], x_off[g - g2 + 1] - x_off[g - g2]);
+    uint32_t big = 0;  // W boxes left to M2P
     if (w_gid)
         for (uint32_t b = w_off[i], e = w_off[i + 1]; b < e; b += kHalf) {  // the half stays together
-            const int2 r = b + o < e ? range[w_gid[b + o]] : make_int2(0, 0);
-            const bool take = b + o < e && r.y - r.x <= direct_max;
-            const uint32_t m = half_ballot(take);
+            const int gw = b + o < e ? w_gid[b + o] : -1;
+            const int2 r = gw >= 0 ? range[gw] : make_int2(0, 0);
+            const bool take = gw >= 0 && r.y - r.x <= direct_max;
+            const uint32_t m = half_ballot(take), mb = half_ballot(gw >= 0 && !take);
+            if (gw >= 0 && !take) m2p_gid[w_off[i] + big + half_rank(mb)] = gw;
+            big += __popc(mb);
             if (take) {
                 n_rng[w + half_rank(m)] = r;
                 sum += r.y - r.x;
@@ -389,6 +394,7 @@ __global__ void __launch_bounds__(256) k_ad_near_fill(const int32_t* __restrict_
     if (o == 0) {
         n_sources[i] = sum;
         n_runs[i] = (int32_t)(w - n_off[i]);
+        m2p_count[i] = (int32_t)big;
     }
 }
 
@@ -723,11 +729,14 @@ int build_adaptive(lfmm_ctx* ctx, int leaf_max, Tree& T, int min_leaf_level)
     T.n_rng = take<int2>(A, T.n_total);
     T.n_sources = take<int32_t>(A, nl);
     T.n_runs = take<int32_t>(A, nl);
-    if (!T.u_rng || !T.n_rng || !T.n_sources || !T.n_runs) return LFMM_ERR_NOMEM;
+    T.m2p_gid = take<int32_t>(A, T.x_pairs);
+    T.m2p_count = take<int32_t>(A, nl);
+    if (!T.u_rng || !T.n_rng || !T.n_sources || !T.n_runs || !T.m2p_gid || !T.m2p_count) return LFMM_ERR_NOMEM;
     hipLaunchKernelGGL(k_ad_u_fill, dim3(nblk(nl, kHalves)), dim3(256), 0, st, nbr27, T.leaf_begin, (int)nl, T.u_off, foff,
                        fcnt, fine_leaf, T.u_rng);
     hipLaunchKernelGGL(k_ad_near_fill, dim3(nblk(nl, kHalves)), dim3(256), 0, st, T.leaf_gid, (int)nl, T.u_off, T.u_rng, xo,
-                       T.x_rng, g2, T.w_off, wg, T.range_all, kDirectMax, T.n_off, T.n_rng, T.n_sources, T.n_runs);
+                       T.x_rng, g2, T.w_off, wg, T.range_all, kDirectMax, T.n_off, T.n_rng, T.n_sources, T.n_runs,
+                       T.m2p_gid, T.m2p_count);
     LFMM_HIP(hipGetLastError());
     return LFMM_OK;
 }

@@ -939,12 +939,11 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
         la.nbr_off = T.n_off;
         la.near_total = T.n_sources;
         la.near_runs = T.n_runs;
-        la.box_range = T.range_all;
-        la.direct_max = kDirectMax;
         la.leaf_lvl = T.leaf_lvl;
         la.leaf_gid = T.leaf_gid;
         la.w_off = T.w_off;
-        la.w_gid = T.w_gid;
+        la.w_gid = T.m2p_gid;
+        la.w_count = T.m2p_count;
         la.keys_all = T.keys_all;
         la.outer_all = outer_all;
         la.depth = depth;

@@ -186,6 +186,8 @@ struct Tree {
     int64_t x_pairs = 0;
     uint32_t* w_off = nullptr;        // W lists: [nleaf + 1] offsets into w_gid
     int32_t* w_gid = nullptr;         //   boxes whose multipoles act on the leaf
+    int32_t* m2p_gid = nullptr;       //   those left to M2P, at the same offsets: m2p_count[leaf] of them
+    int32_t* m2p_count = nullptr;
     uint32_t* n_off = nullptr;        // near lists of the pair kernel: [nleaf + 1] offsets into n_rng
     int2* n_rng = nullptr;            //   U, the leaf's X sources, W boxes of <= kDirectMax particles
     int32_t* n_sources = nullptr;     //   [nleaf] particles in the list, and its ranges

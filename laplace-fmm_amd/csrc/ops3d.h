@@ -110,11 +110,10 @@ struct LeafArgs {
     const int32_t* near_total = nullptr;  // per leaf: the sources in its near ranges,
     const int32_t* near_runs = nullptr;   // and its near ranges
     const uint32_t* w_off = nullptr;
-    const int32_t* w_gid = nullptr;
+    const int32_t* w_gid = nullptr;    // the W boxes left to M2P: w_count[leaf] from w_off[leaf] on
+    const int32_t* w_count = nullptr;
     const uint64_t* keys_all = nullptr;
     const double2* outer_all = nullptr;
-    const int2* box_range = nullptr;   // particle range of every box (gid): W boxes of at most
-    int direct_max = 0;                // direct_max particles are in the near lists, not M2P
     int depth = 0;
     int loff[17] = {};
     int local_min = 2;                 // leaves below this level have no local expansion
