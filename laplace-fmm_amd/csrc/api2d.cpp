@@ -33,7 +33,9 @@ static int get_tables2d(lfmm_ctx* ctx, int N, const DevTables2d** out)
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const std::vector<float> m2l32(T.m2l.begin(), T.m2l.end());  // round to nearest
     std::vector<double> zero(2 * N, 0.0);
-    size_t total = al(T.dir_vec.size() * 4) + al(T.class_dirs.size() * 4) + al(m2l32.size() * 4);
+    std::vector<LogEntry2d> pair_log;
+    pack_log_2d(pair_log);
+    size_t total = al(T.dir_vec.size() * 4) + al(T.class_dirs.size() * 4) + al(m2l32.size() * 4) + al(pair_log.size() * sizeof(LogEntry2d));
     for (auto* v : {&K.m2l, &K.src, &K.out, &K.log, &K.m2m, &K.l2l, &K.down, &K.up, &zero}) total += al(v->size() * 8);
     char* blk = nullptr;
     if (hipMalloc(&blk, total) != hipSuccess) return LFMM_ERR_NOMEM;
@@ -61,6 +63,7 @@ static int get_tables2d(lfmm_ctx* ctx, int N, const DevTables2d** out)
     D->t.down = (const double2*)put(K.down.data(), K.down.size() * 8);
     D->t.up = (const double2*)put(K.up.data(), K.up.size() * 8);
     D->t.zero = (const double2*)put(zero.data(), zero.size() * 8);
+    D->t.pair_log = (const LogEntry2d*)put(pair_log.data(), pair_log.size() * sizeof(LogEntry2d));
     D->t.dir_vec = (const int*)put(T.dir_vec.data(), T.dir_vec.size() * 4);
     D->t.class_dirs = (const int*)put(T.class_dirs.data(), T.class_dirs.size() * 4);
     D->t.m2l32 = (const float2*)put(m2l32.data(), m2l32.size() * 4);
@@ -213,7 +216,7 @@ static int fmm2d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3
     la.field = dfield;
     const size_t ev_leaf = nev;
     if (timed) LFMM_HIP(hipEventRecord(ctx_event(ctx, nev++), st));
-    LFMM_HIP(launch_leaf2d(la, st));
+    LFMM_HIP(launch_leaf2d(la, DT->t, st));
     if (timed) LFMM_HIP(hipEventRecord(ctx_event(ctx, nev++), st));
     if (memory == LFMM_MEM_HOST) {
         if (pot_out) LFMM_HIP(hipMemcpyAsync(pot_out, dpot, sizeof(double) * n_out, hipMemcpyDeviceToHost, st));

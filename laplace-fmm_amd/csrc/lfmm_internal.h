@@ -91,6 +91,19 @@ struct Pack2d {
     std::vector<double> down;   // [N] complex (e/2)^k, e = (1 + i)/2 the class 3 child's offset
     std::vector<double> up;     // [N] complex e^-k
 };
+
+// Logarithm table of the 2D pair term: m in [0.709, 1.418) by intervals of
+// 2^13 in the high word of its double, so that 1 lies inside one of them (kLog2dOne,
+// c = 1): log x = e log 2 + log c + log(1 + r) never cancels.  inv = 1/c to 8
+// fractional bits; log c = hi + lo, hi on a grid of 2^-42.
+constexpr int kLog2dEntries = 128;
+constexpr int kLog2dFirst = 0x3fe6b000;  // high word of the first interval's start
+constexpr int kLog2dOne = 74;
+struct LogEntry2d {
+    double hi;
+    float inv, lo;
+};
+void pack_log_2d(std::vector<LogEntry2d>& t);
 void pack_2d(int N, Pack2d& P);
 
 // Dense real form of the M2L operator of direction `dir` (< kNumM2LDirs):

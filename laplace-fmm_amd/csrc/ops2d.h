@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 
+#include "lfmm_internal.h"
+
 namespace lfmm {
 
 // Device copies of Pack2d, and of what the FP32 M2L takes from OpTables2d.
@@ -16,6 +18,7 @@ struct Tables2d {
     const double2* down;
     const double2* up;
     const double2* zero;       // an expansion of zeros
+    const LogEntry2d* pair_log;
     const float2* m2l32;       // [40][N][N] M2L rounded to FP32 (mixed M2L)
     const int* dir_vec;        // [40][2]
     const int* class_dirs;     // [4][27]
@@ -97,6 +100,6 @@ hipError_t launch_m2m2d(const M2M2dArgs& a, const Tables2d& T, hipStream_t st);
 hipError_t launch_m2l2d(int N, M2L2dLevels& a, const Tables2d& T, hipStream_t st);
 hipError_t launch_m2l2d_f32(int N, const M2L2dArgs& a, const Tables2d& T, hipStream_t st);
 hipError_t launch_l2l2d(const L2L2dArgs& a, const Tables2d& T, hipStream_t st);
-hipError_t launch_leaf2d(const Leaf2dArgs& a, hipStream_t st);
+hipError_t launch_leaf2d(const Leaf2dArgs& a, const Tables2d& T, hipStream_t st);
 
 }  // namespace lfmm

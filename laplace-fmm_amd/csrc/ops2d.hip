@@ -318,22 +318,26 @@ __global__ void __launch_bounds__(256) k_m2l2d32(M2L2dArgs a, Tables2d T)
         if (l0 + r < N) out[l0 + r] = acc[r];
 }
 
-// log(x) of a normal x > 0: x = 2^e m, 1 <= m < 2, a table of 128 (1/c, log c)
-// over m with c within 2^-8 of it, and log(1 + r), r = m/c - 1, by its series to
-// r^6 (next term below 2^-58).  One fma rounds r; the result is within about an
-// ulp.  A third of the library function's operations.
-__device__ __forceinline__ double log_tab(double x, const double2* tab)
+// log(x) of a normal x > 0 by a table (P.T.P. Tang, ACM TOMS 16 (1990) 378;
+// pack_log_2d): x = 2^e m, r = m/c - 1 exact but for its last bit, e log 2 + log c
+// exact in its first part, |r| <= 2^-7 and a series to r^7 (the next term is 2^-59
+// of the first).  Within 0.52 ulp everywhere, next to 1 included (1e7 arguments
+// against 113 bits), as the library function, for half its operations.
+__device__ __forceinline__ double log_tab(double x, const LogEntry2d* tab)
 {
-    const int hi = __double2hiint(x);
-    const double m = __hiloint2double((hi & 0xfffff) | 0x3ff00000, __double2loint(x));
-    const double2 t = tab[(hi >> 13) & 127];
-    const double r = fma(m, t.x, -1.0);
-    double p = fma(r, -1.0 / 6.0, 0.2);
+    const int d = __double2hiint(x) - kLog2dFirst, e = d >> 20;
+    const double m = __hiloint2double(__double2hiint(x) - (e << 20), __double2loint(x));
+    const LogEntry2d t = tab[(d >> 13) & (kLog2dEntries - 1)];
+    const double r = fma(m, (double)t.inv, -1.0);
+    double p = fma(r, 1.0 / 7.0, -1.0 / 6.0);
+    p = fma(r, p, 0.2);
     p = fma(r, p, -0.25);
     p = fma(r, p, 1.0 / 3.0);
     p = fma(r, p, -0.5);
-    p = fma(r * r, p, r);
-    return fma((double)((hi >> 20) - 1023), 0.69314718055994530942, t.y + p);
+    // log 2 in two parts: 42 bits, so that its product with e is exact, and the rest
+    const double h = fma((double)e, 0x1.62e42fefa38p-1, t.hi), w = h + r;
+    const double lo = fma((double)e, 0x1.ef35793c7673p-45, ((h - w) + r) + (double)t.lo);
+    return w + fma(r * r, p, lo);
 }
 
 // Pair term of the reference 2D kernels (src/common/simple_math.h:119-128):
@@ -348,13 +352,10 @@ typedef double pt2d __attribute__((ext_vector_type(4)));
 typedef const pt2d __attribute__((address_space(1)))* pt2d_ptr;
 
 template <bool EXCLUDE, bool WIDE>
-__global__ void __launch_bounds__(256) k_leaf2d(Leaf2dArgs a)
+__global__ void __launch_bounds__(256) k_leaf2d(Leaf2dArgs a, Tables2d T)
 {
-    __shared__ double2 tab[128];
-    if (threadIdx.x < 128) {
-        const double inv = 1.0 / (1.0 + ((double)threadIdx.x + 0.5) / 128.0);
-        tab[threadIdx.x] = make_double2(inv, -log(inv));
-    }
+    __shared__ LogEntry2d tab[kLog2dEntries];
+    if (threadIdx.x < kLog2dEntries) tab[threadIdx.x] = T.pair_log[threadIdx.x];
     __syncthreads();
     const int64_t i = xcd_local_block(blockIdx.x, gridDim.x) * (int64_t)blockDim.x + threadIdx.x;
     const int64_t s = min(i, a.n - 1);
@@ -404,10 +405,14 @@ __global__ void __launch_bounds__(256) k_leaf2d(Leaf2dArgs a)
             fx = fma(qi, dx, fx);
             fy = fma(-qi, dy, fy);
         } else {
+            // w / nz: v_rcp_f64 (relative error 4.7e-8) and one Newton step, then
+            // the quotient's own residual: correctly rounded (8.6e9 quotients
+            // compared with the division; w y alone: a quarter were not); the
+            // fixup keeps infinite charges
             double y = __builtin_amdgcn_rcp(nz);
             y = fma(y, fma(-nz, y, 1.0), y);
-            y = fma(y, fma(-nz, y, 1.0), y);
-            const double qi = w * y;
+            const double q0 = w * y;
+            const double qi = __builtin_amdgcn_div_fixup(fma(fma(-nz, q0, w), y, q0), nz, w);
             ph = fma(w, log_tab(nz, tab), ph);
             fx = fma(qi, dx, fx);
             fy = fma(-qi, dy, fy);
@@ -508,16 +513,16 @@ hipError_t launch_m2l2d_f32(int N, const M2L2dArgs& a, const Tables2d& T, hipStr
     }
 }
 
-hipError_t launch_leaf2d(const Leaf2dArgs& a, hipStream_t st)
+hipError_t launch_leaf2d(const Leaf2dArgs& a, const Tables2d& T, hipStream_t st)
 {
     if (a.n <= 0) return hipSuccess;
     const dim3 grid(nblk(a.n, 256)), block(256);
     if (a.wide) {
-        if (a.exclude_self) hipLaunchKernelGGL((k_leaf2d<true, true>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((k_leaf2d<false, true>), grid, block, 0, st, a);
+        if (a.exclude_self) hipLaunchKernelGGL((k_leaf2d<true, true>), grid, block, 0, st, a, T);
+        else hipLaunchKernelGGL((k_leaf2d<false, true>), grid, block, 0, st, a, T);
     } else {
-        if (a.exclude_self) hipLaunchKernelGGL((k_leaf2d<true, false>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((k_leaf2d<false, false>), grid, block, 0, st, a);
+        if (a.exclude_self) hipLaunchKernelGGL((k_leaf2d<true, false>), grid, block, 0, st, a, T);
+        else hipLaunchKernelGGL((k_leaf2d<false, false>), grid, block, 0, st, a, T);
     }
     return hipGetLastError();
 }

@@ -18,6 +18,7 @@
 
 #include <cmath>
 #include <complex>
+#include <cstring>
 
 namespace lfmm {
 
@@ -155,6 +156,23 @@ void pack_2d(int N, Pack2d& P)
         P.down[2 * k + 1] = (double)a.imag();
         P.up[2 * k] = (double)b.real();
         P.up[2 * k + 1] = (double)b.imag();
+    }
+}
+
+void pack_log_2d(std::vector<LogEntry2d>& t)
+{
+    auto start = [](int i) {
+        const uint64_t u = (uint64_t)(uint32_t)(kLog2dFirst + i * 0x2000) << 32;
+        double v;
+        std::memcpy(&v, &u, sizeof v);
+        return v;
+    };
+    t.resize(kLog2dEntries);
+    for (int i = 0; i < kLog2dEntries; ++i) {
+        const double inv = i == kLog2dOne ? 1.0 : std::rint(512.0 / (start(i) + start(i + 1))) / 256.0;
+        const ld log_c = -std::log((ld)inv);
+        const double hi = std::ldexp(std::rint(std::ldexp((double)log_c, 42)), -42);
+        t[i] = {hi, (float)inv, (float)(log_c - hi)};
     }
 }
 
