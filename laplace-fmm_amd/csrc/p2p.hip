@@ -17,7 +17,8 @@
 // longest leaf total, on a uniform count: per source one compare (the range's
 // end), one pointer step and two loads.  The bounds of the next range are
 // loaded a range ahead; a lane past its list reads a zero charge, so nothing
-// is masked.
+// is masked.  That record sits in its own leaf (pad): far from it, at the origin
+// say, r^2 could overflow, and 0 times that sum's NaN would enter the results.
 #include "device_common.h"
 #include "ops3d.h"
 #include "tree.h"
@@ -41,11 +42,12 @@ __device__ __forceinline__ double rsqrt_nf(double r2)
 
 // Every WIDTH leaves are ordered by the sources of their near lists, so that
 // the leaves of a wave end together: leaf l is pos[l] in lane order,
-// cnt[pos]: its lanes.
+// cnt[pos]: its lanes.  pad[l]: a zero charge at leaf l's first particle.
 template <int TPL, int WIDTH>
 __global__ void __launch_bounds__(512) k_pair_counts(const int32_t* __restrict__ leaf_begin,
                                                     const int32_t* __restrict__ near_total, int nleaf,
-                                                    uint32_t* __restrict__ cnt, int32_t* __restrict__ pos)
+                                                    uint32_t* __restrict__ cnt, int32_t* __restrict__ pos,
+                                                    const double4* __restrict__ src, double4* __restrict__ pad)
 {
     __shared__ uint64_t key[512];
     const int base = blockIdx.x * blockDim.x, l = base + threadIdx.x;
@@ -70,6 +72,8 @@ __global__ void __launch_bounds__(512) k_pair_counts(const int32_t* __restrict__
         leaf = base + (int)(uint32_t)key[threadIdx.x];
     }
     if (l >= nleaf) return;
+    const double4 first = src[leaf_begin[l]];
+    pad[l] = make_double4(first.x, first.y, first.z, 0.0);
     pos[leaf] = l;
     cnt[l] = (uint32_t)((leaf_begin[leaf + 1] - leaf_begin[leaf] + TPL - 1) / TPL);
 }
@@ -87,8 +91,6 @@ __global__ void __launch_bounds__(256) k_pair_lanes(const int32_t* __restrict__ 
     const int64_t k = s - leaf_begin[leaf];
     if (k % TPL == 0) lanes[slot_begin[pos[leaf]] + k / TPL] = (int32_t)s;
 }
-
-__device__ const double kZeroRecord[4] = {0.0, 0.0, 0.0, 0.0};
 
 // a source record, read by global (not flat) loads
 typedef double rec4 __attribute__((ext_vector_type(4)));
@@ -127,7 +129,7 @@ template <int TPL>
 __global__ void __launch_bounds__(256) k_p2p_multi(LeafArgs a, const int32_t* __restrict__ lanes,
                                                   const uint32_t* __restrict__ slot_begin,
                                                   const uint32_t* __restrict__ cnt, int parts,
-                                                  double4* __restrict__ part_out)
+                                                  const double4* __restrict__ pad, double4* __restrict__ part_out)
 {
     const int blk = xcd_local_block(blockIdx.x, gridDim.x);
     const int part = blk % parts;
@@ -167,7 +169,7 @@ __global__ void __launch_bounds__(256) k_p2p_multi(LeafArgs a, const int32_t* __
     // sources of the wave's longest list
     for (int off = 32; off > 0; off >>= 1) nsrc = max(nsrc, __shfl_xor(nsrc, off));
     nsrc = __builtin_amdgcn_readfirstlane(nsrc);
-    const rec4_ptr src = (rec4_ptr)(uintptr_t)a.src, zero = (rec4_ptr)(uintptr_t)&kZeroRecord[0];
+    const rec4_ptr src = (rec4_ptr)(uintptr_t)a.src, zero = (rec4_ptr)(uintptr_t)(pad + leaf);
     rec4_ptr p = zero, end = zero;  // the lane's current range; before the first: at its end
     int64_t step = sizeof(rec4);
     int k = 0, todo = left;  // ranges taken, sources not yet in a taken range
@@ -189,7 +191,7 @@ __global__ void __launch_bounds__(256) k_p2p_multi(LeafArgs a, const int32_t* __
                 end = p + len;
                 todo -= len;
                 rn = nr[min(++k, nrc - 1)];
-            } else {  // past its list: the zero record from here on
+            } else {  // past its list: the leaf's zero charge from here on
                 p = zero;
                 end = src;  // never reached: the step is 0
                 step = 0;
@@ -275,19 +277,20 @@ static int64_t p2p_head_elems(int64_t n, int64_t nleaf) { return (lane_bound(n, 
 int64_t p2p_ws_elems(int64_t n, int64_t nleaf)
 {
     const int parts = p2p_parts(n, nleaf);
-    return p2p_head_elems(n, nleaf) + (parts > 1 ? parts * n * (int64_t)(sizeof(double4) / sizeof(int32_t)) : 0);
+    return p2p_head_elems(n, nleaf) + (nleaf + (parts > 1 ? parts * n : 0)) * (int64_t)(sizeof(double4) / sizeof(int32_t));
 }
 
 template <int TPL>
 static hipError_t p2p_launch(const LeafArgs& a, int32_t* ws, uint32_t* scan_ws, hipStream_t st)
 {
-    // ws: cnt, slot_begin, pos [nleaf each], lanes [lane_bound], then the parts' sums
+    // ws: cnt, slot_begin, pos [nleaf each], lanes [lane_bound], then pad [nleaf] and the parts' sums
     uint32_t* cnt = (uint32_t*)ws;
     uint32_t* slot = cnt + a.nleaf;
     int32_t* pos = (int32_t*)(slot + a.nleaf);
     int32_t* lanes = pos + a.nleaf;
     const int parts = p2p_parts(a.n, a.nleaf);
-    double4* part_out = parts > 1 ? (double4*)(ws + p2p_head_elems(a.n, a.nleaf)) : nullptr;
+    double4* pad = (double4*)(ws + p2p_head_elems(a.n, a.nleaf));
+    double4* part_out = parts > 1 ? pad + a.nleaf : nullptr;
     // Leaves ordered by their source counts end together in a wave (lanes in
     // use on 4M uniform particles: 90 -> 97%), at the price of locality:
     // adaptive lists differ most (512: 4M clustered particles 8.7 -> 7.1 ms),
@@ -296,20 +299,24 @@ static hipError_t p2p_launch(const LeafArgs& a, int32_t* ws, uint32_t* scan_ws, 
     // unordered, 4.9 with 32, 6.2 with 256), or none (64 leaves).
     const dim3 grid(nblk(a.nleaf, 512)), block(512);
     if (a.nbr_off)
-        hipLaunchKernelGGL((k_pair_counts<TPL, 512>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos);
+        hipLaunchKernelGGL((k_pair_counts<TPL, 512>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos,
+                           a.src, pad);
     else if (a.nleaf >= 2048)
-        hipLaunchKernelGGL((k_pair_counts<TPL, 256>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos);
+        hipLaunchKernelGGL((k_pair_counts<TPL, 256>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos,
+                           a.src, pad);
     else if (a.nleaf >= 256)
-        hipLaunchKernelGGL((k_pair_counts<TPL, 32>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos);
+        hipLaunchKernelGGL((k_pair_counts<TPL, 32>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos,
+                           a.src, pad);
     else
-        hipLaunchKernelGGL((k_pair_counts<TPL, 1>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos);
+        hipLaunchKernelGGL((k_pair_counts<TPL, 1>), grid, block, 0, st, a.leaf_begin, a.near_total, a.nleaf, cnt, pos,
+                           a.src, pad);
     hipError_t e = exclusive_scan(cnt, slot, a.nleaf, scan_ws, st);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((k_pair_lanes<TPL>), dim3(nblk(a.n, 256)), dim3(256), 0, st, a.leaf_of, a.leaf_begin, pos, slot,
                        a.n, lanes);
     const int64_t bound = lane_bound(a.n, a.nleaf, TPL);
     hipLaunchKernelGGL((k_p2p_multi<TPL>), dim3(nblk(bound, 256) * parts), dim3(256), 0, st, a, lanes, slot, cnt, parts,
-                       part_out);
+                       pad, part_out);
     if (parts > 1) hipLaunchKernelGGL(k_p2p_join, dim3(nblk(a.n, 256)), dim3(256), 0, st, a, part_out, parts);
     return hipGetLastError();
 }
