@@ -198,11 +198,13 @@ static int fmm2d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3
     int2* nbr = take<int2>(A, T.cnt[leaf_level] * 9);
     int32_t* near_total = take<int32_t>(A, T.cnt[leaf_level]);
     int32_t* near_runs = take<int32_t>(A, T.cnt[leaf_level]);
-    if (!nbr || !near_total || !near_runs) return LFMM_ERR_NOMEM;
+    double4* pad = take<double4>(A, T.cnt[leaf_level]);
+    if (!nbr || !near_total || !near_runs || !pad) return LFMM_ERR_NOMEM;
     LFMM_HIP(launch_leaf_ranges(2, la.leaf_key, la.leaf_begin, la.nleaf, leaf_level,
                                 (leaf_level >= 2 && leaf_level <= lut_max_level(2)) ? T.lut[leaf_level] : nullptr, nbr,
-                                near_total, near_runs, st));
+                                near_total, near_runs, st, T.src, pad));
     la.nbr = nbr;
+    la.pad = pad;
     la.near_total = near_total;
     la.near_runs = near_runs;
     la.wide = scale > 1e150;

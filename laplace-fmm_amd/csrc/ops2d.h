@@ -84,6 +84,7 @@ struct Leaf2dArgs {
     const int2* nbr;           // near-source ranges, 9 entries per leaf
     const int32_t* near_total; // their particles
     const int32_t* near_runs;  // and how many there are
+    const double4* pad;        // per leaf: a zero charge at its first particle
     bool wide;                 // squared distances may overflow
     const double2* local;      // normalised locals of the leaves, or null
     int N;

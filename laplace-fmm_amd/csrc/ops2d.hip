@@ -344,10 +344,11 @@ __device__ __forceinline__ double log_tab(double x, const LogEntry2d* tab)
 // q log(max(|dz|, 1e-4)) and q conj(dz) / max(|dz|^2, 1e-8), self pair included.
 // Bound by vector issue.  A lane walks the near ranges of its leaf as one list
 // (leaves of a wave would wait for each other at every range), one source
-// ahead; past its end it reads a zero charge.  1M particles, 16 per leaf,
+// ahead; past its end it reads a zero charge in its own leaf (at the origin, say,
+// the squared distance could overflow, and 0 times its logarithm is no zero).  1M particles, 16 per leaf,
 // 150M pairs: 0.76 ms with the library's log and division and a loop per
-// neighbour, 0.25 so.  WIDE: distances whose square overflows.
-__device__ const double kZero2d[4] = {0.0, 0.0, 0.0, 0.0};
+// neighbour, 0.25 so.  WIDE: distances whose square overflows, within a leaf too: a
+// lane past its list adds nothing.
 typedef double pt2d __attribute__((ext_vector_type(4)));
 typedef const pt2d __attribute__((address_space(1)))* pt2d_ptr;
 
@@ -364,10 +365,11 @@ __global__ void __launch_bounds__(256) k_leaf2d(Leaf2dArgs a, Tables2d T)
     const int leaf = a.leaf_of[s];
     const double4 t = a.src[s];
     double ph = 0.0, fx = 0.0, fy = 0.0;
-    int todo = live ? a.near_total[leaf] : 0, nsrc = todo;
+    const int all = live ? a.near_total[leaf] : 0;
+    int todo = all, nsrc = all;
     for (int off = 32; off > 0; off >>= 1) nsrc = max(nsrc, __shfl_xor(nsrc, off));
     nsrc = __builtin_amdgcn_readfirstlane(nsrc);
-    const pt2d_ptr src = (pt2d_ptr)(uintptr_t)a.src, zero = (pt2d_ptr)(uintptr_t)&kZero2d[0];
+    const pt2d_ptr src = (pt2d_ptr)(uintptr_t)a.src, zero = (pt2d_ptr)(uintptr_t)(a.pad + leaf);
     const int2* nr = a.nbr + (int64_t)leaf * 9;
     const int nrc = a.near_runs[leaf];
     pt2d_ptr p = zero, end = zero;
@@ -400,6 +402,7 @@ __global__ void __launch_bounds__(256) k_leaf2d(Leaf2dArgs a, Tables2d T)
         q = next();
         const double nz = fmax(fma(dx, dx, dy * dy), 1.e-8);
         if constexpr (WIDE) {
+            if (it >= all) continue;
             const double qi = w / nz;
             ph += w * log(nz);
             fx = fma(qi, dx, fx);

@@ -79,9 +79,11 @@ hipError_t count_ops(int dim, const std::vector<uint64_t*>& keys, const std::vec
                      int64_t* m2l_ops, int64_t* p2p_pairs, int64_t* m2l_per_level, hipStream_t st,
                      int64_t* p2p_reads = nullptr);
 // nbr[leaf][0 .. runs[leaf]) (3^dim entries per leaf) = particle ranges of the
-// neighbour leaves, joined where they touch; total[leaf] their particles
+// neighbour leaves, joined where they touch; total[leaf] their particles;
+// pad[leaf] (optional) = a zero charge at the leaf's first particle
 hipError_t launch_leaf_ranges(int dim, const uint64_t* leaf_key, const int32_t* leaf_begin, int nleaf, int level,
-                              const int32_t* lut, int2* nbr, int32_t* total, int32_t* runs, hipStream_t st);
+                              const int32_t* lut, int2* nbr, int32_t* total, int32_t* runs, hipStream_t st,
+                              const double4* src = nullptr, double4* pad = nullptr);
 // p[0..n) = v with a fill kernel (safe inside stream capture)
 hipError_t fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t st);
 }  // namespace lfmm

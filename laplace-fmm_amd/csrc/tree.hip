@@ -555,7 +555,8 @@ template <int D>
 __global__ void __launch_bounds__(256) k_leaf_ranges(const uint64_t* __restrict__ leaf_key,
                                                      const int32_t* __restrict__ leaf_begin, int nleaf, int level,
                                                      const int32_t* __restrict__ lut, int2* __restrict__ nbr,
-                                                     int32_t* __restrict__ total, int32_t* __restrict__ nruns)
+                                                     int32_t* __restrict__ total, int32_t* __restrict__ nruns,
+                                                     const double4* __restrict__ src, double4* __restrict__ pad)
 {
     constexpr int G = D == 3 ? 32 : 16, K = D == 3 ? 27 : 9;
     __shared__ int2 sorted[256 / G][G];
@@ -604,6 +605,10 @@ __global__ void __launch_bounds__(256) k_leaf_ranges(const uint64_t* __restrict_
     if (o == 0) {
         total[leaf] = sum;
         nruns[leaf] = __popc(heads);
+        if (pad) {
+            const double4 first = src[leaf_begin[leaf]];
+            pad[leaf] = make_double4(first.x, first.y, first.z, 0.0);
+        }
     }
     const int run = __popc(heads & ((2u << o) - 1u)) - 1;
     if (head) out[2 * run] = r.x;
@@ -762,14 +767,15 @@ hipError_t count_ops(int dim, const std::vector<uint64_t*>& keys, const std::vec
 }
 
 hipError_t launch_leaf_ranges(int dim, const uint64_t* leaf_key, const int32_t* leaf_begin, int nleaf, int level,
-                              const int32_t* lut, int2* nbr, int32_t* total, int32_t* runs, hipStream_t st)
+                              const int32_t* lut, int2* nbr, int32_t* total, int32_t* runs, hipStream_t st,
+                              const double4* src, double4* pad)
 {
     if (nleaf > 0 && dim == 2)
         hipLaunchKernelGGL(k_leaf_ranges<2>, dim3(nblk(nleaf, 16)), dim3(256), 0, st, leaf_key, leaf_begin, nleaf, level, lut,
-                           nbr, total, runs);
+                           nbr, total, runs, src, pad);
     else if (nleaf > 0)
         hipLaunchKernelGGL(k_leaf_ranges<3>, dim3(nblk(nleaf, 8)), dim3(256), 0, st, leaf_key, leaf_begin, nleaf, level, lut,
-                           nbr, total, runs);
+                           nbr, total, runs, src, pad);
     return hipGetLastError();
 }
 
