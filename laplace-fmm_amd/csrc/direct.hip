@@ -30,13 +30,14 @@ __device__ __forceinline__ double rsqrt_full(double r2)
     return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-// All pairs.  A workgroup of 1024 threads owns 2 LT targets, two per lane
-// (LT lanes), and cuts the sources into 1024 / LT interleaved slices, one per
-// group of LT lanes; the slices' sums are added in a fixed order at the end
-// (shuffles within a wave, then LDS over the waves).  So few targets still
-// fill the chip without a buffer for partial sums: one thread per target ran
-// 4,096 targets on 16 of 256 CUs (123 ms against 1,048,576 sources).
-// Bound by FP64 vector issue: 23 operations and v_rsq_f64 per 3D pair.  With
+// All pairs, targets first .. end - 1.  A workgroup of 1024 threads owns 2 LT of
+// them, two per lane (LT lanes), and cuts the sources into 1024 / LT interleaved
+// slices, one per group of LT lanes; the slices' sums are added in a fixed order
+// at the end (shuffles within a wave, then LDS over the waves).  So 512 targets
+// and more fill the chip without a buffer for partial sums: one thread per target
+// ran 4,096 targets on 16 of 256 CUs (123 ms against 1,048,576 sources).  Fewer
+// than 512 leave CUs idle.
+// Bound by FP64 vector issue: 19 operations and v_rsq_f64 per 3D pair.  With
 // LT >= 64 a wave's source is uniform and arrives by scalar loads; below, two
 // targets per lane halve the L1 reads per pair, which one target per lane
 // would be bound by (64 lanes x 32 bytes at 64 bytes per cycle).
@@ -76,8 +77,8 @@ struct DirectSum<2> {
 constexpr int kDirectThreads = 1024;
 
 template <int DIM, int LT, bool EXCLUDE>
-__global__ void __launch_bounds__(kDirectThreads) k_direct(const double4* __restrict__ tgt, int64_t nt,
-                                                          const double4* __restrict__ src, int64_t ns,
+__global__ void __launch_bounds__(kDirectThreads) k_direct(const double4* __restrict__ tgt, int64_t first,
+                                                          int64_t end, const double4* __restrict__ src, int64_t ns,
                                                           double* __restrict__ pot, double* __restrict__ field)
 {
     constexpr int S = kDirectThreads / LT, NW = kDirectThreads / 64;
@@ -90,8 +91,8 @@ __global__ void __launch_bounds__(kDirectThreads) k_direct(const double4* __rest
     DirectSum<DIM> a[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-        i[u] = (int64_t)blockIdx.x * (2 * LT) + u * LT + lt;
-        t[u] = i[u] < nt ? tgt[i[u]] : make_double4(0.0, 0.0, 0.0, 0.0);
+        i[u] = first + (int64_t)blockIdx.x * (2 * LT) + u * LT + lt;
+        t[u] = i[u] < end ? tgt[i[u]] : make_double4(0.0, 0.0, 0.0, 0.0);
     }
     auto pair = [&](int64_t j, double sx, double sy, double sz, double q) {
 #pragma unroll
@@ -142,7 +143,7 @@ __global__ void __launch_bounds__(kDirectThreads) k_direct(const double4* __rest
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-        if (i[u] >= nt) continue;
+        if (i[u] >= end) continue;
         if (pot) pot[i[u]] = a[u].p;
         if (field) {
             field[DIM * i[u]] = a[u].fx;
@@ -238,30 +239,54 @@ hipError_t launch_cross_fields(const double* e1, const double* e2, double* e3, i
 }
 
 template <int DIM, int LT>
-static hipError_t direct_lt(const double4* tgt, int64_t nt, const double4* src, int64_t ns, bool exclude, double* pot,
-                            double* field, hipStream_t st)
+static hipError_t direct_lt(const double4* tgt, int64_t first, int64_t end, const double4* src, int64_t ns, bool exclude,
+                            double* pot, double* field, hipStream_t st)
 {
-    const dim3 grid((unsigned)((nt + 2 * LT - 1) / (2 * LT)));
+    const dim3 grid((unsigned)((end - first + 2 * LT - 1) / (2 * LT))), block(kDirectThreads);
     if (exclude)
-        hipLaunchKernelGGL((k_direct<DIM, LT, true>), grid, dim3(kDirectThreads), 0, st, tgt, nt, src, ns, pot, field);
+        hipLaunchKernelGGL((k_direct<DIM, LT, true>), grid, block, 0, st, tgt, first, end, src, ns, pot, field);
     else
-        hipLaunchKernelGGL((k_direct<DIM, LT, false>), grid, dim3(kDirectThreads), 0, st, tgt, nt, src, ns, pot, field);
+        hipLaunchKernelGGL((k_direct<DIM, LT, false>), grid, block, 0, st, tgt, first, end, src, ns, pot, field);
     return hipGetLastError();
 }
+
+// A CU holds one workgroup (126 registers, 1024 threads), so the targets go in
+// rounds of 256 workgroups, and a round that is not full takes as long as a full
+// one.  Each launch therefore takes whole rounds at the largest LT that fills
+// one, and what is left goes on in smaller rounds, down to 512 targets, unless
+// less than a launch's time is gained.  One launch at one LT lost up to half:
+// 200,000 sources and 530,000 targets 149 -> 76 ms (one thread per target:
+// 99), 270,000 75 -> 38 (59), 4,097 1.36 -> 0.86 (4,096: 0.78).
+constexpr int64_t kDirectRound = 512;      // targets of a round at LT = 1
+constexpr int64_t kDirectGain = 8000000;   // pairs in 8 us (2D: 28 us)
 
 template <int DIM>
 static hipError_t direct_dim(const double4* tgt, int64_t nt, const double4* src, int64_t ns, bool exclude, double* pot,
                              double* field, hipStream_t st)
 {
-    // the most targets per workgroup that still give every CU one workgroup
-    int lt = 1;
-    while (lt < kDirectThreads && nt >= (int64_t)256 * 2 * (2 * lt)) lt *= 2;
-    switch (lt) {
-#define X(n) case n: return direct_lt<DIM, n>(tgt, nt, src, ns, exclude, pot, field, st);
-        X(1) X(2) X(4) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
+    int least = 1;  // no more slices than there are sources for
+    while (least < kDirectThreads && kDirectThreads / least > ns) least *= 2;
+    for (int64_t at = 0; at < nt;) {
+        const int64_t left = nt - at;
+        int lt = least;
+        while (lt < kDirectThreads && left >= kDirectRound * 2 * lt) lt *= 2;
+        const int64_t round = kDirectRound * lt, rest = left % round;
+        int64_t end = nt;
+        if (left > round && rest > 0) {
+            const int64_t small = kDirectRound * least;
+            const int64_t gained = round - rest - (small - rest % small) % small;
+            if (gained > kDirectGain / std::max<int64_t>(ns, 1)) end = nt - rest;
+        }
+        hipError_t e = hipErrorInvalidValue;
+        switch (lt) {
+#define X(n) case n: e = direct_lt<DIM, n>(tgt, at, end, src, ns, exclude, pot, field, st); break;
+            X(1) X(2) X(4) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
 #undef X
-    default: return hipErrorInvalidValue;
+        }
+        if (e != hipSuccess) return e;
+        at = end;
     }
+    return hipSuccess;
 }
 
 hipError_t launch_direct(int dim, const double4* tgt, int64_t nt, const double4* src, int64_t ns, bool exclude_self,
