@@ -29,7 +29,7 @@ static int get_tables2d(lfmm_ctx* ctx, int N, const DevTables2d** out)
     OpTables2d T;
     build_op_tables_2d(N, T);
     Pack2d K;
-    pack_2d(N, K);
+    pack_2d(T, K);
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const std::vector<float> m2l32(T.m2l.begin(), T.m2l.end());  // round to nearest
     std::vector<double> zero(2 * N, 0.0);

@@ -103,6 +103,7 @@ void check_tables_2d()
     for (int N = 1; N <= LFMM_MAX_TERMS_2D; ++N) {
         lfmm::OpTables2d T;
         lfmm::build_op_tables_2d(N, T);
+        lfmm::build_shift_tables_2d(T);
         expect(T.m2l.size() == (size_t)lfmm::kNumM2LDirs2d * N * N * 2, "2d m2l size", N);
         for (double v : T.m2l) expect(std::isfinite(v), "2d m2l finite", N);
         for (double v : T.m2m) expect(std::isfinite(v), "2d m2m finite", N);

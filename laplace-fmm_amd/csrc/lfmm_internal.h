@@ -75,6 +75,8 @@ struct OpTables2d {
     std::vector<double> l2l;       // [4][N][N] complex (child class c)
 };
 void build_op_tables_2d(int N, OpTables2d& T);
+// m2m and l2l: what the factored forms are checked against, in no solve
+void build_shift_tables_2d(OpTables2d& T);
 
 // Factored form of the 2D operators, every entry a real matrix between two
 // complex diagonals (see pack_2d); complex values interleaved.
@@ -104,7 +106,7 @@ struct LogEntry2d {
     float inv, lo;
 };
 void pack_log_2d(std::vector<LogEntry2d>& t);
-void pack_2d(int N, Pack2d& P);
+void pack_2d(const OpTables2d& T, Pack2d& P);
 
 // Dense real form of the M2L operator of direction `dir` (< kNumM2LDirs):
 // K[row * N^2 + col], rows and columns in m2l_real_index order.

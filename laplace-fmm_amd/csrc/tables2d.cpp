@@ -40,6 +40,12 @@ static cld cpow_l(cld z, int e)
     return r;
 }
 
+static void put(std::vector<double>& v, size_t i, cld z)
+{
+    v[2 * i] = (double)z.real();
+    v[2 * i + 1] = (double)z.imag();
+}
+
 // child class c = (x bit << 1) | y bit of the child's Morton key
 static cld child_offset(int c) { return cld((c & 2) ? 0.5L : -0.5L, (c & 1) ? 0.5L : -0.5L); }
 
@@ -64,24 +70,28 @@ void build_op_tables_2d(int N, OpTables2d& T)
             T.class_dirs[c * kDirsPerClass2d + cnt++] = d;
         }
     }
-    auto put = [](std::vector<double>& v, size_t i, cld z) {
-        v[2 * i] = (double)z.real();
-        v[2 * i + 1] = (double)z.imag();
-    };
     T.m2l.assign((size_t)ND * N * N * 2, 0.0);
+    std::vector<cld> pw(2 * N);  // z^k
     for (int d = 0; d < ND; ++d) {
         const cld z((ld)T.dir_vec[2 * d], (ld)T.dir_vec[2 * d + 1]);
+        pw[0] = 1;
+        for (int k = 1; k < 2 * N; ++k) pw[k] = pw[k - 1] * z;
         for (int l = 0; l < N; ++l)
             for (int j = 0; j < N; ++j) {
                 cld v;
                 const ld sj = (j & 1) ? -1.0L : 1.0L;
                 if (l == 0 && j == 0) v = std::conj(std::log(-z));
-                else if (l == 0) v = sj / cpow_l(z, j);
-                else if (j == 0) v = -1.0L / ((ld)l * cpow_l(z, l));
-                else v = sj * binom_l(l + j - 1, j - 1) / cpow_l(z, l + j);
+                else if (l == 0) v = sj / pw[j];
+                else if (j == 0) v = -1.0L / ((ld)l * pw[l]);
+                else v = sj * binom_l(l + j - 1, j - 1) / pw[l + j];
                 put(T.m2l, ((size_t)d * N + l) * N + j, v);
             }
     }
+}
+
+void build_shift_tables_2d(OpTables2d& T)
+{
+    const int N = T.N;
     T.m2m.assign((size_t)4 * N * N * 2, 0.0);
     T.l2l.assign((size_t)4 * N * N * 2, 0.0);
     for (int c = 0; c < 4; ++c) {
@@ -110,10 +120,9 @@ void build_op_tables_2d(int N, OpTables2d& T)
 // i^r e, so a child enters M2M as i^(r (j-s)), which depends on (j - s) mod 4
 // alone: the children's four sums with weights i^(r m) go through one real
 // matrix, and the L2L is the transpose.
-void pack_2d(int N, Pack2d& P)
+void pack_2d(const OpTables2d& T, Pack2d& P)
 {
-    OpTables2d T;
-    build_op_tables_2d(N, T);
+    const int N = T.N;
     const int ND = (int)T.dir_vec.size() / 2, NB = m2l2d_blocks(N), pairs = m2l2d_pairs(N), regs = m2l2d_regs(N);
     P.m2l.assign((size_t)NB * regs * 16, 0.0);
     for (int l = 0; l < N; ++l)
