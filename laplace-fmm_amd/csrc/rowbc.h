@@ -1,7 +1,10 @@
 // rowbc.h -- FP64 products with a coefficient broadcast from a register that
 // holds 16 of them, one per lane of each 16-lane row (row_newbcast, full rate;
 // the compiler does not fold the broadcast into the product).  The coefficient
-// register is to be written by a load, not by a vector instruction just before.
+// register is to be written by a load: less than 2 wait states after a vector
+// instruction wrote it the broadcast would read the old value, and the compiler,
+// which cannot see into the assembly, may copy or reload a spilled register there.
+// check_dpp.py looks for that in every built library.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <type_traits>
