@@ -1246,7 +1246,7 @@ static int tree_export_adaptive(lfmm_ctx* c, const lfmm_points3d* particles, int
         if (w_box)
             for (int64_t k = 0; k < T.x_pairs; ++k) w_box[k] = wg[k];
         if (x_off) {
-            for (int gi = 0; gi <= total; ++gi) x_off[gi] = gi < g2 ? 0 : (int64_t)xo[gi - g2];
+            for (int gi = 0; gi <= total; ++gi) x_off[gi] = gi < g2 || xo.empty() ? 0 : (int64_t)xo[gi - g2];  // two levels: no X lists
         }
         if (x_leaf)
             for (int64_t k = 0; k < T.x_pairs; ++k) x_leaf[k] = leaf_at(xrng[k].x);
