@@ -61,17 +61,18 @@ __device__ inline int ad_cover(const AdLevels& A, int l, int x, int y, int z)
 
 // The uniform levels the adaptive tree is cut from, concatenated: level l's
 // boxes are off[l] .. off[l + 1] - 1, its begin and first arrays (one entry
-// more per level) start at off[l] + l.
+// more per level) start at off[l] + l.  All levels together can hold several
+// times the particles (a deep tree of a dense clump in an even background).
 struct UniLevels {
     int depth;
-    int off[kAdMaxLevels + 1];
+    int64_t off[kAdMaxLevels + 1];
     const uint64_t* keys;
     const int32_t* child;
     const int32_t* first;
     const int32_t* parent;
 };
 
-__device__ inline int uni_level(const UniLevels& U, int j)
+__device__ inline int uni_level(const UniLevels& U, int64_t j)
 {
     int l = 0;
     while (l + 1 < U.depth && j >= U.off[l + 1]) ++l;
@@ -94,7 +95,7 @@ struct AdKeep {
     __device__ uint32_t operator()(int64_t j) const
     {
         if (j >= U.off[U.depth]) return 0u;
-        const int l = uni_level(U, (int)j);
+        const int l = uni_level(U, j);
         if (l == 0 || l <= min_leaf_level) return 1u;
         const int32_t* f = U.first + U.off[l - 1] + (l - 1) + U.parent[j];
         return f[1] - f[0] > leaf_max ? 1u : 0u;
@@ -120,7 +121,7 @@ __global__ void __launch_bounds__(256) k_ad_fill(UniLevels U, AdLevels A, const 
                                                  int2* __restrict__ range_all, int32_t* __restrict__ child,
                                                  int32_t* __restrict__ box2leaf, int32_t* __restrict__ tag)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (j < U.depth) child[A.off[j + 1] + j] = j + 1 < U.depth ? A.off[j + 2] - A.off[j + 1] : 0;
     if (j >= U.off[U.depth]) return;
     const int g = (int)kex[j];
@@ -569,8 +570,8 @@ int build_adaptive(lfmm_ctx* ctx, int leaf_max, Tree& T, int min_leaf_level)
     // ---- kept boxes and their numbering
     UniLevels U{};
     U.depth = depth;
-    for (int l = 0; l < depth; ++l) U.off[l + 1] = U.off[l] + (int)T.cnt[l];
-    const int utotal = U.off[depth];
+    for (int l = 0; l < depth; ++l) U.off[l + 1] = U.off[l] + T.cnt[l];
+    const int64_t utotal = U.off[depth];
     U.keys = T.lkeys[0];
     U.child = T.lbegin[0];
     U.first = T.ufirst[0];

@@ -265,6 +265,7 @@ int build_tree(lfmm_ctx* ctx, const DevPoints& DP, int depth_in, int leaf_max, b
     const int dim = DP.dim;
     hipStream_t st = ctx->stream;
     Arena& A = ctx->arena;
+    if (n > kMaxTreeParticles) return LFMM_ERR_HIP;
     T.n = n;
     T.dim = dim;
     const double* dpos = DP.pos;

@@ -20,6 +20,7 @@
 
 namespace lfmm::host {
 
+constexpr int64_t kMaxTreeParticles = (int64_t)1 << 28;  // lists and lanes are sized and tested up to here
 constexpr int kMaxDepth = 16;   // 15 bits per axis at the leaves (3D)
 // dense key -> box tables up to 2^24 entries (levels <= 8 in 3D, <= 12 in 2D)
 constexpr int lut_max_level(int dim) { return 24 / dim; }

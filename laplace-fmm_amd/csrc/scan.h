@@ -140,7 +140,7 @@ template <typename In, typename Out>
 hipError_t scan_apply(In in, Out out, int64_t n, uint32_t* ws, hipStream_t st)
 {
     const int64_t nb = (n + kScanTile - 1) / kScanTile;
-    if (n < 0 || nb > 1024 * 64) return hipErrorInvalidValue;
+    if (n < 0 || nb >= (int64_t)1 << 22) return hipErrorInvalidValue;  // 2^32 threads in a launch
     if (nb == 0) return hipSuccess;
     const dim3 grid((unsigned)nb), block(kScanThreads);
     if (nb > 1) hipLaunchKernelGGL((k_scan_reduce<In>), grid, block, 0, st, in, n, ws);
