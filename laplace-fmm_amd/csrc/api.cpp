@@ -701,7 +701,8 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
         for (int l = first; l < (mixed ? std::min(mfl, depth) : depth); ++l)
             if (cnt[l] >= kPackMinBoxes && cnt[l] >= (int64_t)kPackMinFill * cnt[l - 1])
                 big = std::max<int64_t>(big, m2lv_slots(cnt[l - 1]));
-        if (big > 0 && !(vpack = take<double2>(A, 8 * NX * big))) return LFMM_ERR_NOMEM;
+        // a quarter more memory than the solve needs otherwise: without it the M2L reads the boxes themselves
+        if (big > 0) vpack = (double2*)A.try_alloc((size_t)(8 * NX * big) * sizeof(double2));
     }
     // sources of an adaptive level packed by the parents with children alone
     // (4M clustered particles: a quarter of all; packing 0.80 -> 0.34 ms, whole
@@ -730,8 +731,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
             const bool bucketed = adaptive && l >= mfl && (per_box || cnt[l - 1] >= kBucketMinParents);
             // FP64 M2L of a large, mostly full level: sources class-major
             double2* vpacked = nullptr;
-            if (!(mixed && l >= mfl) && !per_box && N <= kM2lvMaxTerms && cnt[l] >= kPackMinBoxes &&
-                cnt[l] >= (int64_t)kPackMinFill * cnt[l - 1]) {
+            if (vpack && !(mixed && l >= mfl) && cnt[l] >= kPackMinBoxes && cnt[l] >= (int64_t)kPackMinFill * cnt[l - 1]) {
                 vpacked = vpack;
                 LFMM_HIP(launch_m2lv_pack(L, NX, vpacked, st));
             }

@@ -68,6 +68,19 @@ struct Arena {
         peak = std::max(peak, used);
         return p;
     }
+    // alloc for a buffer that the caller can do without: on failure the arena
+    // stays as it was (alloc leaves what is left of its chunks) and so does HIP's error
+    void* try_alloc(size_t bytes)
+    {
+        const size_t cur0 = cur, off0 = off;
+        void* p = alloc(bytes);
+        if (!p) {
+            cur = cur0;
+            off = off0;
+            (void)hipGetLastError();
+        }
+        return p;
+    }
     void release()
     {
         for (auto& c : chunks) (void)hipFree(c.p);

@@ -1,7 +1,8 @@
 // host_check.cpp -- exercises the host-side C++ of the library without a
 // GPU: the FP64 table builders (3D and 2D), their packed forms unpacked again
-// as the kernels read them, the dense and split-fp16 M2L operators, the exact-file reader and writer, ReadError's statistics, and
-// the argument checks every entry point runs before device work.  Built
+// as the kernels read them, the dense and split-fp16 M2L operators, the arena,
+// the exact-file reader and writer, ReadError's statistics, and the argument
+// checks every entry point runs before device work.  Built
 // together with the library's host sources under AddressSanitizer and
 // UndefinedBehaviorSanitizer (make sanitize); any report aborts the run.
 // Prints "host_check ok" and exits 0 when every check holds.
@@ -13,6 +14,7 @@
 #include <vector>
 
 #include "lfmm.h"
+#include "api_internal.h"
 #include "lfmm_internal.h"
 #include "m2l64.h"
 #include "m2lv.h"
@@ -371,6 +373,18 @@ void check_exact_files(const std::string& dir)
     expect(lfmm_error_stats(7, 1, nullptr, nullptr, nullptr, nullptr, nullptr) != LFMM_OK, "stats bad kind");
 }
 
+// A buffer that cannot be had leaves the arena's next allocation where it was.
+void check_arena()
+{
+    std::vector<char> mem(4096);
+    lfmm::host::Arena A;
+    A.chunks.push_back({mem.data(), mem.size()});
+    expect(A.alloc(1000) == mem.data(), "arena first");
+    expect(A.try_alloc((size_t)1 << 60) == nullptr, "arena too large");
+    expect(A.try_alloc(1000) == mem.data() + 1024 && A.alloc(2048) == mem.data() + 2048, "arena goes on");
+    expect(A.used == 4096 && A.peak == 4096, "arena use");
+}
+
 // Entry points given a null context fail with LFMM_ERR_INVALID before any
 // device work.
 void check_null_context()
@@ -408,6 +422,7 @@ int main(int argc, char** argv)
     check_packed_3d();
     check_tables_2d();
     check_exact_files(dir);
+    check_arena();
     check_null_context();
     if (failures) {
         std::printf("host_check: %d failures\n", failures);
