@@ -5,8 +5,10 @@
 // tables on the device, and the launch sequence
 //   extent -> keys -> radix sort -> gather -> levels -> P2M -> M2M (up)
 //   -> M2L+L2L (down) -> P2P+L2P (leaves, scattered to input order).
-// Everything runs on one HIP stream; the only host synchronisations are the
-// box counts of each level (needed to size the next launch).
+// Everything runs on one HIP stream.  The host waits where a size decides the
+// next allocation or launch: once per sort of the tree build (one, two or three;
+// see build_tree), three times for the lists of an adaptive tree, and for the
+// order buckets.
 #include "api_internal.h"
 #include "direct.h"
 
@@ -550,17 +552,17 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
     if (mixed) {
         rc = get_m16(ctx, N, &DT);
         if (rc != LFMM_OK) return rc;
-        // packed sources of the largest mixed level: box-major (size + 1
-        // boxes) or class-major (8 classes x (parents + 1) slots)
+        // packed sources of the largest mixed level, class-major (8 classes x
+        // (parents + 1) slots)
         int64_t big = 0;
         for (int l = mfl; l < depth; ++l)
-            big = std::max(big, m16_rowfull(N) ? 8 * (cnt[l - 1] + 1) : cnt[l] + 1);
+            big = std::max(big, 8 * (cnt[l - 1] + 1));
         const int64_t nr = (int64_t)N * N, pieces = (nr + 15) / 16 * 4;
         xp = take<uint4>(A, big * pieces);
         xmax = take<uint32_t>(A, depth);
         if (!xp || !xmax) return LFMM_ERR_NOMEM;
         LFMM_HIP(fill_u32(xmax, depth, 0u, st));
-        if (!adaptive && m16_rowfull(N)) {
+        if (!adaptive) {
             // uniform tree: every matrix-core level packed once, when its
             // multipoles are final, for its M2M into the level above and its
             // own M2L
@@ -803,7 +805,7 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                             m.ctile[c + 1] = m.ctile[c] + (m.coff[c + 1] - m.coff[c] + m16_targets(t) - 1) / m16_targets(t);
                         m.tiles = m.ctile[8];
                         m.xpieces = 4 * ((tpack * tpack + 15) / 16);
-                        if (m16_rowfull(tpack)) slots_of(m, l);
+                        slots_of(m, l);
                         // a workgroup runs all 189 directions of its targets:
                         // small buckets split the directions into parts so
                         // that about 512 workgroups share the work
@@ -856,12 +858,10 @@ int fmm3d_solve(lfmm_ctx* ctx, const lfmm_points3d* S, const lfmm_points3d* Tg, 
                 m.kinv = DT->m16_kinv;
                 m.dst = inner[l];
                 m.tiles = (int)((cnt[l - 1] + m16_targets(N) - 1) / m16_targets(N));
-                // the row-complete kernel holds one workgroup per CU: about
-                // 256 workgroups, one wave of them (measured 0.13 ms faster
-                // over levels 4-5 at 13 terms than 512: fewer parts to sum)
-                m.dsplit = m16_rowfull(N) ? (int)std::max<int64_t>(1, std::min<int64_t>(32, (256 + m.tiles * 8 - 1) /
-                                                                                                 (m.tiles * 8)))
-                                          : dsplit_for((int64_t)m.tiles * 8);
+                // one workgroup fits a CU: about 256 workgroups, one wave of
+                // them (measured 0.13 ms faster over levels 4-5 at 13 terms
+                // than 512: fewer parts to sum)
+                m.dsplit = (int)std::max<int64_t>(1, std::min<int64_t>(32, (256 + m.tiles * 8 - 1) / (m.tiles * 8)));
                 if (m.dsplit > 1) {
                     // every part writes its whole slice (no clearing needed)
                     m.partial = take<double2>(A, (int64_t)m.dsplit * cnt[l] * NX);

@@ -289,10 +289,10 @@ int order_leaf_terms_from_requests(hipStream_t st, const Tree& T, const int32_t*
                                    uint32_t* leaf_terms);
 // Box terms and the (level, terms) launch buckets of the boxes of levels >= first_bucket_level.  promote:
 // buckets of few boxes take the next larger order of their level (fewer launches).  Synchronises.
-// The same for one order everywhere: plist and seg by class alone.
-int order_class_lists(lfmm_ctx* ctx, const Tree& T, int terms, int first_bucket_level, BoxOrders& O);
 int order_box_terms(lfmm_ctx* ctx, const Tree& T, const uint32_t* leaf_terms, int first_bucket_level, BoxOrders& O,
                     bool promote = false);
+// The same for one order everywhere: plist and seg by class alone.
+int order_class_lists(lfmm_ctx* ctx, const Tree& T, int terms, int first_bucket_level, BoxOrders& O);
 // Algorithmic FP64 flops of all M2L operations at their orders (levels below
 // first_bucket_level at N).  Synchronises.
 int order_m2l_flops(lfmm_ctx* ctx, const Tree& T, const BoxOrders& O, int N, int first_bucket_level, double* flops);

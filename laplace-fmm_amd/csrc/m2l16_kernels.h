@@ -21,8 +21,8 @@
 // the FP64 L2L of the parent.
 //
 // Operands (32x32x16 f16 MFMA; lane l, slot s in 0..7):
-//   A  row l % 32, K index 8 * (l / 32) + s     (operator, from global/L2)
-//   B  col l % 32, K index 8 * (l / 32) + s     (sources, staged in LDS)
+//   A  row l % 32, K index 8 * (l / 32) + s     (operator, through LDS)
+//   B  col l % 32, K index 8 * (l / 32) + s     (sources, from global/L2)
 //   C  col l % 32, row 8 * (v / 4) + 4 * (l / 32) + v % 4, v = 0..15
 // A and B use the same (lane, slot) -> K assignment, so the sum over K does
 // not depend on how the hardware numbers K within an instruction.
@@ -46,7 +46,6 @@ struct M16 {
     static constexpr int NR = N * N;            // real coordinates of an expansion
     static constexpr int RT = (NR + 31) / 32;   // row tiles of 32
     static constexpr int KC = (NR + 15) / 16;   // K chunks of 16
-    static constexpr int RW = (RT + 3) / 4;     // row tiles per wave (at most)
     static constexpr int PIECES = KC * 4;       // 16-byte pieces of a packed source box
 };
 
@@ -67,35 +66,6 @@ __device__ inline int m16_coef_offset(int r)
     const int m = (q + 1) >> 1;
     const int part = (q != 0 && !(q & 1)) ? 1 : 0;
     return 2 * (tri(n) + m) + part;
-}
-
-// Packs a level's normalised multipoles into the B operand layout:
-// [box][KC][part hi/lo][half][8 x fp16]; box `size` is all zeros.
-template <int N>
-__global__ void __launch_bounds__(256) k_m2l16_pack(const double2* __restrict__ outer, int size,
-                                                    const uint32_t* __restrict__ xmax, uint4* __restrict__ xp)
-{
-    using S = M16<N>;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;  // (box, kc, half)
-    if (i >= (int64_t)(size + 1) * S::KC * 2) return;
-    const int half = (int)(i & 1);
-    const int kc = (int)((i >> 1) % S::KC);
-    const int64_t box = (i >> 1) / S::KC;
-    const double sc = m16_xscale(*xmax);
-    const double* src = (const double*)(outer + box * tri(N));
-    m16_h8 hv, lv;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        const int k = kc * 16 + half * 8 + s;
-        double x = 0.0;
-        if (box < size && k < S::NR) x = src[m16_coef_offset(k)] * sc;
-        const _Float16 h = (_Float16)x;
-        hv[s] = h;
-        lv[s] = (_Float16)(x - (double)h);
-    }
-    uint4* dst = xp + (box * S::KC + kc) * 4;
-    dst[half] = __builtin_bit_cast(uint4, hv);
-    dst[2 + half] = __builtin_bit_cast(uint4, lv);
 }
 
 // Packs a level's normalised multipoles class-major for k_m2l16r:
@@ -168,250 +138,7 @@ __global__ void __launch_bounds__(256) k_m2l16_pack_cls(const double2* __restric
 // and sparse; below 12 terms the straight-line MFMA stream is faster.
 constexpr bool m16_skip(int N) { return N >= 12; }
 
-template <int N, int CT>
-__global__ void __launch_bounds__(256) k_m2l16(M2L16Args a, const uint4* __restrict__ kmat, const uint4* __restrict__ xp,
-                                               const int* __restrict__ class_dirs, const int* __restrict__ dir_vec,
-                                               const int2* __restrict__ kpre)
-{
-    using S = M16<N>;
-    constexpr int RT = S::RT, KC = S::KC, RW = S::RW, NR = S::NR, PIECES = S::PIECES;
-    constexpr int TC = 32 * CT;        // targets (columns) per workgroup
-    constexpr int TPC = 256 / TC;      // loader threads per column
-    constexpr int PPT = (PIECES + TPC - 1) / TPC;  // 16-byte pieces per loader thread
-    static_assert(256 % TC == 0, "loader split");
-    __shared__ uint4 bs[2][CT][KC][2][64];
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform
-    // row tiles w, w + 4, ... of this wave; all valid when RT divides over the 4 waves
-    constexpr bool kEven = (RT % 4) == 0;
-    const int blk = xcd_local_block(blockIdx.x, gridDim.x);
-    // tile-major block order: the 8 child classes (and direction parts) of a
-    // tile are adjacent, so the workgroups of one XCD read overlapping sources
-    const int tile = blk / (8 * a.dsplit);
-    const int part = (blk - tile * 8 * a.dsplit) >> 3;
-    const int c = blk & 7;
-    const int d_beg = part * kDirsPerClass / a.dsplit, d_end = (part + 1) * kDirsPerClass / a.dsplit;
-    const int side = 1 << a.level;
-
-    // target box of column `col`: the class-c child of parent tile * TC + col
-    auto target_of = [&](int col, uint32_t& x, uint32_t& y, uint32_t& z) -> int {
-        const int P = tile * TC + col;
-        int t = -1;
-        if (P < a.num_parents) {
-            const int cb = a.child_begin[P], ce = a.child_begin[P + 1];
-            for (int i = cb; i < ce; ++i)
-                if ((int)(a.child_keys[i] & 7u) == c) t = i;
-        }
-        if (t >= 0) {
-            const uint64_t k = a.child_keys[t];
-            x = compact3(k >> 2);
-            y = compact3(k >> 1);
-            z = compact3(k);
-        }
-        return t;
-    };
-
-    // ---- B staging: loader thread (column lcol, part lq) moves PPT pieces
-    const int lcol = tid / TPC, lq = tid % TPC;
-    uint32_t lx = 0, ly = 0, lz = 0;
-    const int ltgt = target_of(lcol, lx, ly, lz);
-    auto source_piece = [&](int d) -> const uint4* {
-        const int dir = class_dirs[c * kDirsPerClass + d];
-        int box = a.size;  // the zero box
-        if (ltgt >= 0) {
-            const int sx = (int)lx + dir_vec[4 * dir], sy = (int)ly + dir_vec[4 * dir + 1],
-                      sz = (int)lz + dir_vec[4 * dir + 2];
-            if (sx >= 0 && sy >= 0 && sz >= 0 && sx < side && sy < side && sz < side) {
-                const int s = find_box(morton3(sx, sy, sz), a.lut, a.keys, a.size);
-                if (s >= 0) box = s;
-            }
-        }
-        return xp + (int64_t)box * PIECES + lq;
-    };
-    auto stage_slot = [&](int buf, int i) -> uint4* {
-        const int pc = lq + TPC * i;
-        return &bs[buf][lcol >> 5][pc >> 2][(pc >> 1) & 1][(pc & 1) * 32 + (lcol & 31)];
-    };
-    constexpr bool kFullPieces = (PIECES % TPC) == 0;
-    auto piece_ok = [&](int i) { return kFullPieces || lq + TPC * i < PIECES; };
-    // Operator fragments of this wave's row tiles stream through a rolling
-    // window: chunk kc + LA is loaded while chunk kc is multiplied (across the
-    // step boundary into the next direction).  Only the blocks the precision
-    // needs are loaded and multiplied: per (direction, row tile), chunks
-    // kc < k3 use hi*hi + hi*lo + lo*hi, k3 <= kc < k1 hi*hi alone, the rest
-    // nothing (host table kpre; see pack_m2l16).
-    // one row tile per wave: the whole next step is prefetched; two: 4 chunks ahead
-    constexpr int LA = RW == 1 ? KC : 4;
-    auto dir_of = [&](int d) { return class_dirs[c * kDirsPerClass + d]; };
-    auto row_tile = [&](int r) { return kEven ? w + 4 * r : min(w + 4 * r, RT - 1); };
-    auto prefix = [&](int dir, int r) -> int2 {
-        if (!kEven && w + 4 * r >= RT) return make_int2(0, 0);
-        if constexpr (!m16_skip(N)) return make_int2(KC, KC);
-        const int2 v = kpre[dir * RT + row_tile(r)];
-        // wave-uniform: keep the block bounds in scalar registers (scalar branches)
-        return make_int2(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y));
-    };
-    // unneeded fragments are read from one fixed block (cache-resident), so
-    // every load is unconditional and the loop stays straight-line code
-    auto frag = [&](int dir, int r, int kc, int hl, bool need) -> uint4 {
-        const int64_t blk = need ? (int64_t)dir * (RT * KC * 2) + (row_tile(r) * KC + kc) * 2 + hl : 0;
-        return kmat[blk * 64 + lane];
-    };
-
-    m16_acc acc[RW][CT];
-#pragma unroll
-    for (int r = 0; r < RW; ++r)
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[r][ct][v] = 0.0f;
-
-    // step d_beg: sources staged, first LA operator chunks loaded
-    int dcur = dir_of(d_beg);
-    int2 pc[RW];
-    uint4 hh[RW][LA], hl[RW][LA];
-#pragma unroll
-    for (int r = 0; r < RW; ++r) {
-        pc[r] = prefix(dcur, r);
-#pragma unroll
-        for (int k = 0; k < LA; ++k) {
-            hh[r][k] = frag(dcur, r, k, 0, k < pc[r].y);
-            hl[r][k] = frag(dcur, r, k, 1, k < pc[r].x);
-        }
-    }
-    {
-        const uint4* p = source_piece(d_beg);
-        uint4 t[PPT];
-#pragma unroll
-        for (int i = 0; i < PPT; ++i) t[i] = piece_ok(i) ? p[TPC * i] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < PPT; ++i)
-            if (piece_ok(i)) *stage_slot(0, i) = t[i];
-    }
-    lds_barrier();
-    for (int d = d_beg; d < d_end; ++d) {
-        const int buf = (d - d_beg) & 1;
-        const int dn = min(d + 1, d_end - 1);  // the last step re-stages its own data (never read)
-        const int dnext = dir_of(dn);
-        int2 pn[RW];
-#pragma unroll
-        for (int r = 0; r < RW; ++r) pn[r] = prefix(dnext, r);
-        // next step's sources, in flight under the MFMAs
-        uint4 nb[PPT];
-        {
-            const uint4* p = source_piece(dn);
-#pragma unroll
-            for (int i = 0; i < PPT; ++i) nb[i] = piece_ok(i) ? p[TPC * i] : make_uint4(0, 0, 0, 0);
-        }
-        uint4 ch[RW][KC], cl[RW][KC];  // this step's chunks LA.. (loaded LA chunks ahead)
-        uint4 nh[RW][LA], nl[RW][LA];  // next step's chunks 0..LA-1
-        uint4 fb[2][CT][2];
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            fb[0][ct][0] = bs[buf][ct][0][0][lane];
-            fb[0][ct][1] = bs[buf][ct][0][1][lane];
-        }
-#pragma unroll
-        for (int kc = 0; kc < KC; ++kc) {
-            // issue the operator chunk LA ahead
-            const int ka = kc + LA;
-#pragma unroll
-            for (int r = 0; r < RW; ++r) {
-                if (ka < KC) {
-                    ch[r][ka] = frag(dcur, r, ka, 0, ka < pc[r].y);
-                    cl[r][ka] = frag(dcur, r, ka, 1, ka < pc[r].x);
-                } else {
-                    nh[r][ka - KC] = frag(dnext, r, ka - KC, 0, ka - KC < pn[r].y);
-                    nl[r][ka - KC] = frag(dnext, r, ka - KC, 1, ka - KC < pn[r].x);
-                }
-            }
-            // source fragments of chunk kc + 1 are read while chunk kc multiplies
-            if (kc + 1 < KC) {
-#pragma unroll
-                for (int ct = 0; ct < CT; ++ct) {
-                    fb[(kc + 1) & 1][ct][0] = bs[buf][ct][kc + 1][0][lane];
-                    fb[(kc + 1) & 1][ct][1] = bs[buf][ct][kc + 1][1][lane];
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < RW; ++r) {
-                const uint4 ah = kc < LA ? hh[r][kc] : ch[r][kc];
-                const uint4 al = kc < LA ? hl[r][kc] : cl[r][kc];
-                const m16_h8 xh = __builtin_bit_cast(m16_h8, ah);
-                const m16_h8 xl = __builtin_bit_cast(m16_h8, al);
-                if (kc < pc[r].y) {
-#pragma unroll
-                    for (int ct = 0; ct < CT; ++ct) {
-                        const m16_h8 bh = __builtin_bit_cast(m16_h8, fb[kc & 1][ct][0]);
-                        acc[r][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, bh, acc[r][ct], 0, 0, 0);
-                    }
-                }
-                if (kc < pc[r].x) {
-#pragma unroll
-                    for (int ct = 0; ct < CT; ++ct) {
-                        const m16_h8 bl = __builtin_bit_cast(m16_h8, fb[kc & 1][ct][1]);
-                        acc[r][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, bl, acc[r][ct], 0, 0, 0);
-                    }
-#pragma unroll
-                    for (int ct = 0; ct < CT; ++ct) {
-                        const m16_h8 bh = __builtin_bit_cast(m16_h8, fb[kc & 1][ct][0]);
-                        acc[r][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, bh, acc[r][ct], 0, 0, 0);
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < PPT; ++i)
-            if (piece_ok(i)) *stage_slot(buf ^ 1, i) = nb[i];
-#pragma unroll
-        for (int r = 0; r < RW; ++r) {
-            pc[r] = pn[r];
-#pragma unroll
-            for (int k = 0; k < LA; ++k) {
-                hh[r][k] = nh[r][k];
-                hl[r][k] = nl[r][k];
-            }
-        }
-        dcur = dnext;
-        lds_barrier();
-    }
-
-    // ---- epilogue: L += acc / (scale of K * scale of X), in FP64 (or the
-    // part's partial sum, summed into L by a reduction, when split)
-    const double inv = a.kinv / m16_xscale(*a.xmax);
-    double2* const dst = a.dsplit > 1 ? a.partial + (int64_t)part * a.size * tri(N) : a.dst;
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-        uint32_t tx, ty, tz;
-        const int t = target_of(ct * 32 + (lane & 31), tx, ty, tz);
-        if (t < 0) continue;
-        double* out = (double*)(dst + (int64_t)t * tri(N));
-        if (a.dsplit > 1 && w == 0) {
-            // the part's slice is written whole: the imaginary parts of the
-            // m = 0 coefficients (no real coordinate) as zeros; lanes l and
-            // l + 32 hold the same target
-            for (int n = lane >> 5; n < N; n += 2) out[2 * tri(n) + 1] = 0.0;
-        }
-#pragma unroll
-        for (int r = 0; r < RW; ++r) {
-            const int rt = w + 4 * r;
-            if (!kEven && rt >= RT) continue;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int row = rt * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-                if (row < NR) {
-                    const int o = m16_coef_offset(row);
-                    const double val = (double)acc[r][ct][v] * inv;
-                    if (a.dsplit > 1) out[o] = val;
-                    else out[o] += val;
-                }
-            }
-        }
-    }
-}
-
-// ===================================================================== row-complete variant
+// ===================================================================== the M2L
 // k_m2l16r: every wave computes all row tiles of its own CTW column tiles, so
 // the four waves of a workgroup need the same operator fragments and share
 // them through LDS; each wave loads its own source fragments straight into
@@ -421,7 +148,7 @@ __global__ void __launch_bounds__(256) k_m2l16(M2L16Args a, const uint4* __restr
 // registers) while segment i is multiplied and written to the other LDS
 // buffer afterwards: one barrier per segment, no wave waits for another's
 // rows, and each operator fragment read from LDS feeds 2 * CTW or 4 * CTW
-// MFMAs.  Skipping is per (direction, row tile), as in k_m2l16: hi*hi below
+// MFMAs.  Skipping is per (direction, row tile; host table kpre, see pack_m2l16): hi*hi below
 // the tile's k1, hi*lo + lo*hi below its k3, under scalar branches on the
 // wave-uniform bounds (at 13 terms 96 instead of 131 MFMAs per direction and
 // column tile, averaged over the directions the classes use); the sources
@@ -819,35 +546,25 @@ __global__ void __launch_bounds__(256, CTW == 1 ? 2 : 1) k_m2l16r(M2L16Args a, c
         if (a.absmax) wave_absmax(mx, a.absmax);
 }
 
-// Targets per workgroup = 32 * m16_ct(N): two column tiles while the
-// double-buffered source stage (64 KiB per tile at N = 16) fits the LDS.
-constexpr int m16_ct(int N) { return N <= 16 ? 2 : 1; }
-
 template <int N>
 hipError_t do_m2l16_pack(const M2L16Args& a, hipStream_t st)
 {
-    if constexpr (m16_rowfull(N)) {
-        const int parents = a.slot ? a.slots : a.num_parents;
-        const int64_t packs = ((int64_t)parents + 1) * M16<N>::KC * 2;
-        hipLaunchKernelGGL((k_m2l16_pack_cls<N>), dim3((unsigned)((packs + 255) / 256)), dim3(256), 0, st, a.outer,
-                           parents, a.child_begin, a.child_keys, a.xmax, a.xp,
-                           (int64_t)(a.stride > 0 ? a.stride : tri(N)), a.slot ? a.slot_parents : nullptr);
-    } else {
-        const int64_t packs = (int64_t)(a.size + 1) * M16<N>::KC * 2;
-        hipLaunchKernelGGL((k_m2l16_pack<N>), dim3((unsigned)((packs + 255) / 256)), dim3(256), 0, st, a.outer,
-                           a.size, a.xmax, a.xp);
-    }
+    const int parents = a.slot ? a.slots : a.num_parents;
+    const int64_t packs = ((int64_t)parents + 1) * M16<N>::KC * 2;
+    hipLaunchKernelGGL((k_m2l16_pack_cls<N>), dim3((unsigned)((packs + 255) / 256)), dim3(256), 0, st, a.outer,
+                       parents, a.child_begin, a.child_keys, a.xmax, a.xp,
+                       (int64_t)(a.stride > 0 ? a.stride : tri(N)), a.slot ? a.slot_parents : nullptr);
     return hipGetLastError();
 }
 
 template <int N>
 hipError_t do_m2l16(const M2L16Args& a, hipStream_t st)
 {
-    static_assert(m16_targets(N) == (m16_rowfull(N) ? 128 * m16r_ctw(N) : 32 * m16_ct(N)), "tile width");
+    static_assert(m16_targets(N) == 128 * m16r_ctw(N), "tile width");
     const int targets = a.plist ? a.plist_count : a.num_parents;
     const int tiles = (targets + m16_targets(N) - 1) / m16_targets(N);
     if (a.csorted) {
-        if (!a.plist || a.dsplit < 1 || a.dsplit > kDirsPerClass || !m16_rowfull(N) || a.coff[8] != a.plist_count ||
+        if (!a.plist || a.dsplit < 1 || a.dsplit > kDirsPerClass || a.coff[8] != a.plist_count ||
             (a.dsplit > 1 && !a.partial))
             return hipErrorInvalidValue;
         for (int c = 0; c < 8; ++c)
@@ -855,26 +572,20 @@ hipError_t do_m2l16(const M2L16Args& a, hipStream_t st)
                 return hipErrorInvalidValue;
         int mt = 0;
         for (int c = 0; c < 8; ++c) mt = mt > a.ctile[c + 1] - a.ctile[c] ? mt : a.ctile[c + 1] - a.ctile[c];
-        if constexpr (m16_rowfull(N))
-            if (mt > 0)
-                hipLaunchKernelGGL((k_m2l16r<N, m16r_ctw(N)>), dim3(8 * mt * a.dsplit), dim3(256), 0, st, a, a.kmat,
-                                   (const uint4*)a.xp, a.class_dirs, a.dir_vec, a.kpre);
+        if (mt > 0)
+            hipLaunchKernelGGL((k_m2l16r<N, m16r_ctw(N)>), dim3(8 * mt * a.dsplit), dim3(256), 0, st, a, a.kmat,
+                               (const uint4*)a.xp, a.class_dirs, a.dir_vec, a.kpre);
         return hipGetLastError();
     }
     if (tiles != a.tiles || a.dsplit < 1 || a.dsplit > kDirsPerClass) return hipErrorInvalidValue;
-    if (a.m2m && (!m16_rowfull(N) || a.dsplit != 1 || a.plist || a.stride || a.src_np1 < 1)) return hipErrorInvalidValue;
-    if (a.plist && (a.dsplit != 1 || !m16_rowfull(N))) return hipErrorInvalidValue;
+    if (a.m2m && (a.dsplit != 1 || a.plist || a.stride || a.src_np1 < 1)) return hipErrorInvalidValue;
+    if (a.plist && a.dsplit != 1) return hipErrorInvalidValue;
     if (tiles > 0) {
-        if constexpr (m16_rowfull(N)) {
-            if (a.m2m)
-                hipLaunchKernelGGL((k_m2l16r<N, m16r_ctw(N), true>), dim3(tiles * 8), dim3(256), 0, st, a, a.kmat,
-                                   (const uint4*)a.xp, a.class_dirs, a.dir_vec, a.kpre);
-            else
-                hipLaunchKernelGGL((k_m2l16r<N, m16r_ctw(N)>), dim3(tiles * 8 * a.dsplit), dim3(256), 0, st, a, a.kmat,
-                                   (const uint4*)a.xp, a.class_dirs, a.dir_vec, a.kpre);
-        }
+        if (a.m2m)
+            hipLaunchKernelGGL((k_m2l16r<N, m16r_ctw(N), true>), dim3(tiles * 8), dim3(256), 0, st, a, a.kmat,
+                               (const uint4*)a.xp, a.class_dirs, a.dir_vec, a.kpre);
         else
-            hipLaunchKernelGGL((k_m2l16<N, m16_ct(N)>), dim3(tiles * 8 * a.dsplit), dim3(256), 0, st, a, a.kmat,
+            hipLaunchKernelGGL((k_m2l16r<N, m16r_ctw(N)>), dim3(tiles * 8 * a.dsplit), dim3(256), 0, st, a, a.kmat,
                                (const uint4*)a.xp, a.class_dirs, a.dir_vec, a.kpre);
     }
     return hipGetLastError();

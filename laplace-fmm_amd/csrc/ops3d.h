@@ -128,8 +128,7 @@ struct M2L16Args {
     const uint4* kmat;         // split-fp16 operator fragments [dir][RT][KC][2][64]
     const int2* kpre;          // [dir][RT] (k3, k1): K chunks needing all products / hi*hi
     const double2* outer;      // normalised multipoles of the level
-    uint4* xp;                 // packed sources: k_m2l16 [size + 1][KC][2][2] (box `size` is zero);
-                               // k_m2l16r [8 classes][KC][2][2][num_parents + 1] (slot num_parents is zero)
+    uint4* xp;                 // packed sources: [8 classes][KC][2][2][num_parents + 1] (slot num_parents is zero)
     const uint32_t* xmax;      // largest |coefficient| of the level (float bits)
     const int* class_dirs;
     const int* dir_vec;
@@ -185,19 +184,13 @@ struct M2L16Args {
     uint32_t* absmax = nullptr;
 };
 
-// Matrix-core M2L kernel per expansion size: the row-complete k_m2l16r
-// (operator shared through LDS, 128 or 256 targets per workgroup) from
-// LFMM_M16R_MIN_N terms on, below it k_m2l16 (sources shared through LDS, 64
-// or 32 targets per workgroup).
-#ifndef LFMM_M16R_MIN_N
-#define LFMM_M16R_MIN_N 1
-#endif
-constexpr bool m16_rowfull(int N) { return N >= LFMM_M16R_MIN_N; }
+// Matrix-core M2L: the operator shared through LDS, 128 or 256 targets per
+// workgroup.
 // k_m2l16r keeps two column tiles per wave up to this many row tiles of 32
 constexpr int m16r_max_rt2 = 6;
 constexpr int m16_targets(int N)
 {
-    return m16_rowfull(N) ? ((N * N + 31) / 32 <= m16r_max_rt2 ? 256 : 128) : (N <= 16 ? 64 : 32);
+    return (N * N + 31) / 32 <= m16r_max_rt2 ? 256 : 128;
 }
 
 hipError_t launch_p2m(int N, const P2MArgs& a, hipStream_t st);
@@ -206,12 +199,12 @@ hipError_t launch_p2l(int N, const P2MArgs& a, hipStream_t st);
 // M2M (kind 0) and L2L (2) from LFMM_RTR_MIN_N terms on; below, launch_m2lv
 #define LFMM_RTR_MIN_N 14
 hipError_t launch_rtr(int N, int kind, const RtrTables& T, const RtrLevel& L, hipStream_t st);
-// L2P alone into a.far (k_l2p), for the pair kernels below
 // M2M of the listed parents, split over parts: part p of list entry i is at
 // partial + (p * count + i) * nx, their sum goes to dst + list[i] * nx (and its
 // largest |coefficient| to absmax)
 hipError_t launch_sum_parent_parts(const double2* partial, int parts, int count, int nx, const int32_t* list, double2* dst,
                                    uint32_t* absmax, hipStream_t st);
+// L2P alone into a.far (k_l2p), for the pair kernels below
 hipError_t launch_l2p(int N, const LeafArgs& a, hipStream_t st);
 // Near field with several targets per lane (p2p.hip), starting from a.far when
 // set.  ws: p2p_ws_elems(n, nleaf) int32; scan_ws: scan_ws_elems(nleaf).
