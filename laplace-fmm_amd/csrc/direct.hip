@@ -250,9 +250,9 @@ static hipError_t direct_lt(const double4* tgt, int64_t first, int64_t end, cons
     return hipGetLastError();
 }
 
-// A CU holds one workgroup (126 registers, 1024 threads), so the targets go in
-// rounds of 256 workgroups, and a round that is not full takes as long as a full
-// one.  Each launch therefore takes whole rounds at the largest LT that fills
+// A CU holds one workgroup (1024 threads; 3D: 126 registers), so the targets go
+// in rounds of 256 workgroups, and a round that is not full takes as long as a
+// full one.  Each launch therefore takes whole rounds at the largest LT that fills
 // one, and what is left goes on in smaller rounds, down to 512 targets, unless
 // less than a launch's time is gained.  One launch at one LT lost up to half:
 // 200,000 sources and 530,000 targets 149 -> 76 ms (one thread per target:

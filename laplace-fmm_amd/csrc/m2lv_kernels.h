@@ -26,9 +26,9 @@
 // On large, mostly full levels the sources are packed class-major
 // (m2lv_pack.hip): one box per lane costs the L1 64 tag lookups per load.
 //
-// Measured, 4M uniform particles (M2L of all levels, with the packing; before,
-// with scalar operands): 9 terms 8.3 -> 6.8 ms, 11 terms 16.2 -> 11.2 ms, 13
-// terms 49.0 -> 17.2 ms (32 TFLOP/s algorithmic).  The vector units are busy
+// Measured, 4M uniform particles (M2L of all levels; before, with scalar
+// operands): 9 terms 8.3 -> 6.6 ms, 11 terms 16.2 -> 11.0 ms, 13 terms 49.0 -> 16.9
+// ms (33 TFLOP/s algorithmic); the packing adds 0.2 ms.  The vector units are busy
 // about half of the time; the rest is the phase barriers (5%), the source
 // loads (13%) and dependent issue with 2 waves per SIMD.
 #pragma once

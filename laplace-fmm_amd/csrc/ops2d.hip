@@ -152,7 +152,8 @@ __global__ void __launch_bounds__(kPairs2d) k_l2l2d(L2L2dArgs a, Tables2d T)
 // to each, and broadcasts them by row_newbcast.  (As complex entries per
 // direction, read from LDS, it was 4 products and a 16-byte LDS read each, and a
 // launch per level: 1M particles of 21 terms, 0.82 -> 0.22 ms.)  Two row blocks from 12 terms
-// on: more waves, and their accumulators and entries fit beside the source.
+// on and three from 25: more waves, and their accumulators and entries fit beside
+// the source.
 template <int N>
 __global__ void __launch_bounds__(64) k_m2l2d(M2L2dLevels A, Tables2d T)
 {
@@ -322,7 +323,7 @@ __global__ void __launch_bounds__(256) k_m2l2d32(M2L2dArgs a, Tables2d T)
 // pack_log_2d): x = 2^e m, r = m/c - 1 exact but for its last bit, e log 2 + log c
 // exact in its first part, |r| <= 2^-7 and a series to r^7 (the next term is 2^-59
 // of the first).  Within 0.52 ulp everywhere, next to 1 included (1e7 arguments
-// against 113 bits), as the library function, for half its operations.
+// against 113 bits), as the library function, for about half its operations.
 __device__ __forceinline__ double log_tab(double x, const LogEntry2d* tab)
 {
     const int d = __double2hiint(x) - kLog2dFirst, e = d >> 20;
@@ -345,9 +346,10 @@ __device__ __forceinline__ double log_tab(double x, const LogEntry2d* tab)
 // Bound by vector issue.  A lane walks the near ranges of its leaf as one list
 // (leaves of a wave would wait for each other at every range), one source
 // ahead; past its end it reads a zero charge in its own leaf (at the origin, say,
-// the squared distance could overflow, and 0 times its logarithm is no zero).  1M particles, 16 per leaf,
-// 150M pairs: 0.76 ms with the library's log and division and a loop per
-// neighbour, 0.25 so.  WIDE: distances whose square overflows, within a leaf too: a
+// the squared distance could overflow, and 0 times its logarithm is no zero).  1M
+// particles, 16 per leaf, 150M pairs: 0.76 ms with the library's log and division and
+// a loop per neighbour, 0.32 so (0.25 with a logarithm that cancels next to 1 and an
+// uncorrected quotient).  WIDE: distances whose square overflows, within a leaf too: a
 // lane past its list adds nothing.
 typedef double pt2d __attribute__((ext_vector_type(4)));
 typedef const pt2d __attribute__((address_space(1)))* pt2d_ptr;

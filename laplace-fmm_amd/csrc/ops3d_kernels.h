@@ -699,8 +699,8 @@ __global__ void __launch_bounds__(256) k_l2p(LeafArgs a, const double2* __restri
     }
     if constexpr (ADAPTIVE) {
         // most W boxes are summed directly by the pair kernel: these are the
-        // rest (a test per box and lane, each two dependent loads: 7M particles
-        // in 512 systems 1.90 ms, so 1.33)
+        // rest (a test per box and lane, each two dependent loads: 8.5M
+        // particles in 512 systems 1.90 ms, so 1.33)
         const uint32_t wb = a.w_off[leaf], we = wb + (uint32_t)a.w_count[leaf];
         for (uint32_t k = wb; k < we; ++k) {
             const int g = a.w_gid[k];

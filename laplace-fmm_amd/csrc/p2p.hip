@@ -12,7 +12,7 @@
 // per leaf: lane slot_begin[leaf] + k owns targets leaf_begin[leaf] + TPL k ...
 // + TPL k + TPL - 1.
 //
-// Bound by vector issue: 22 FP64 operations and v_rsq_f64 per pair.  A lane
+// Bound by vector issue: 18 FP64 operations and v_rsq_f64 per pair.  A lane
 // walks the near ranges of its leaf as one list, so a wave runs as long as its
 // longest leaf total, on a uniform count: per source one compare (the range's
 // end), one pointer step and two loads.  The bounds of the next range are
@@ -263,8 +263,9 @@ inline int p2p_tpl(int64_t n, int64_t nleaf) { return n >= 64 * nleaf ? 4 : 2; }
 // leave the chip idle (50,000 particles in 64 leaves: 195 waves for 1,024
 // SIMDs; 4.7 ms in one part, 0.6 in 64) or end unevenly (400,000 in 512: 8.6
 // -> 4.9 ms).  16 waves per SIMD keep all of them busy to the end (8: 3% less
-// on 1M particles in 4,096 leaves).  A part has at least 128 sources (256:
-// 65,536 particles in 4,096 leaves 0.081 -> 0.128 ms).
+// on 1M particles in 4,096 leaves).  A part of a list of average length has at
+// least 128 sources (256: 65,536 particles in 4,096 leaves 0.081 -> 0.128 ms); shorter
+// lists are split as often.
 static int p2p_parts(int64_t n, int64_t nleaf)
 {
     const int64_t waves = n / (64 * p2p_tpl(n, nleaf)) + 1;
@@ -293,8 +294,8 @@ static hipError_t p2p_launch(const LeafArgs& a, int32_t* ws, uint32_t* scan_ws, 
     double4* part_out = parts > 1 ? pad + a.nleaf : nullptr;
     // Leaves ordered by their source counts end together in a wave (lanes in
     // use on 4M uniform particles: 90 -> 97%), at the price of locality:
-    // adaptive lists differ most (512: 4M clustered particles 8.7 -> 7.1 ms),
-    // uniform ones less (256: 1.95 -> 1.74 ms); with few, large leaves only
+    // adaptive lists differ most (512: 4M clustered particles 4.3 -> 3.6 ms),
+    // uniform ones less (256: 4M particles 1.95 -> 1.74 ms); with few, large leaves only
     // near neighbours are exchanged (400,000 particles in 512 leaves: 5.4 ms
     // unordered, 4.9 with 32, 6.2 with 256), or none (64 leaves).
     const dim3 grid(nblk(a.nleaf, 512)), block(512);

@@ -451,7 +451,7 @@ __global__ void __launch_bounds__(256) k_level_emit(const uint64_t* __restrict__
 
 // Particles of every leaf in input order, where their order came from keys of
 // a finer level: each moves to its rank among its leaf's.  Most of these leaves
-// hold a few particles (7M of them: 0.74 ms with half a wave per leaf).
+// hold a few particles (8.5M of them: 0.74 ms with half a wave per leaf).
 __global__ void __launch_bounds__(256) k_leaf_order(const int32_t* __restrict__ leaf_of, const int32_t* __restrict__ begin,
                                                     int64_t n, const uint32_t* __restrict__ in, uint32_t* __restrict__ out)
 {

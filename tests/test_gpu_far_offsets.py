@@ -5,7 +5,7 @@ square overflows but no distance within the cloud does.
 1e-130 of it, so the potential is 10^4 q to a few ulp and the field next to
 nothing.  2D: the oracle is the direct sum in long double, every pair near: 1e-8
 (single terms are good to a few ulp).  With a far field the results are only
-asked to be finite: a box's centre is rounded to the coordinates' grid, a 64th
+asked to be finite: a box's centre is rounded to the coordinates' grid, a 256th
 of a leaf here, and so is its accuracy."""
 import numpy as np
 import pytest
